@@ -100,6 +100,7 @@ void awefd_destroy(awefd_model *m)
     free(m->h_rsinc);
     awefd__spher_free(m);
     awefd__adjoint_free(m);
+    awefd__res_free(m);
     if (m->cgexec) hipGraphExecDestroy(m->cgexec);
     if (m->cgraph) hipGraphDestroy(m->cgraph);
     free(m);
@@ -299,7 +300,7 @@ int awefd_create(const awefd_params *p, awefd_model **out)
         return awefd__fail(AWEFD_ENOMEM, "hipMalloc of 3 x %zu bytes: %s", bytes,
                            hipGetErrorString(e));
     }
-    if (!is_cart(m) && (rc = awefd__spher_create(m)) != 0) {
+    if ((rc = is_cart(m) ? awefd__res_create(m) : awefd__spher_create(m)) != 0) {
         awefd_destroy(m);
         return rc;
     }
@@ -658,7 +659,7 @@ static int cart_build_inj(awefd_model *m)
     if (!rc) rc = upload(m, (void **)&m->d_ibeg, ibeg, sizeof(int) * (nbucket + 1));
     m->ninj = n;
     free(e); free(ibeg);
-    return rc;
+    return rc ? rc : awefd__res_set_sources(m);
 }
 
 int awefd_set_sources(awefd_model *m, int ns, const float *coords)
@@ -683,7 +684,7 @@ int awefd_set_receivers(awefd_model *m, int nr, const float *coords)
     if (!rc && m->sinc)
         rc = upload(m, (void **)&m->d_rsinc, m->h_rsinc, sizeof(awefd_sinc_pt) * (nr > 0 ? nr : 1));
     if (!rc && m->inj_rec) rc = cart_build_inj(m);
-    if (!rc && !is_cart(m)) rc = awefd__spher_set_receivers(m);
+    if (!rc) rc = is_cart(m) ? awefd__res_set_receivers(m) : awefd__spher_set_receivers(m);
     if (!rc) m->rec_set = 1;
     const int rd = setter_done(m);
     return rc ? rc : rd;
@@ -1000,7 +1001,8 @@ static int cart_loop(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, vo
     return rc;
 }
 
-/* The 2-D loop as one graph: a 2-D step is a few microseconds of work, so
+/* The 2-D loop as one graph, for the models the resident loop does not hold
+ * (awefd_resident.c): a 2-D step is a few microseconds of work, so
  * per-launch overhead would dominate a stream of nt launches.  Captured when
  * a run repeats the previous one (same model generation and trace buffer;
  * a one-off run is cheaper launched directly), then launched per run; the
@@ -1059,9 +1061,14 @@ static int run_common(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
     if (rc) return rc;
     HIPCHK(hipSetDevice(m->dev));
     if ((rc = awefd__ensure_traces(m))) return rc;
-    if ((rc = awefd_reset(m))) return rc;
     const int plain2d = is_cart(m) && m->ndim == 2 && !m->prof && !(cb && jsnap > 0);
     float *trow0 = dtr ? dtr : m->d_traces;
+    if (plain2d && m->res.on) {
+        /* the resident loop starts from zero fields of its own */
+        int done;
+        if ((rc = awefd__res_run(m, trow0, &done)) || done) return rc;
+    }
+    if ((rc = awefd_reset(m))) return rc;
     const int repeat = plain2d && ((m->cvalid && m->cgen == m->gen && m->cdtr == trow0) ||
                                    (m->eager_seen && m->eager_gen == m->gen && m->eager_dtr == trow0));
     if (repeat) {

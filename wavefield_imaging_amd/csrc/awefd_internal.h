@@ -141,6 +141,66 @@ typedef struct {
     const awefd_rx3 *rx3;
 } awefd_cart_args;
 
+/* The resident 2-D loop (res_loop.h): blocks of AWEFD_RES_NWAVE waves; S
+ * steps per exchange; a tile owns 64 - 2 S nop z nodes of 8 rx - 2 (S - 1)
+ * nop x rows (rx: rows a wave computes). */
+#define AWEFD_RES_NWAVE 8
+#define AWEFD_RES_MAXNOP 4       /* stencil half-widths compiled               */
+typedef struct {
+    int on;                      /* a compiled tile whose blocks fit           */
+    int rx, S;
+    int zw, ox, ntz, ntx;        /* owned nodes of a tile, tiles               */
+    long words;                  /* 64-bit words of a block's rim              */
+} awefd_res_tile;
+typedef struct {
+    int n1, n2, ld;              /* padded grid, row stride                    */
+    int ntz, ntx;                /* tiles                                      */
+    int blk0;                    /* batched: first block of this shot          */
+    int nb, dabc;
+    float c0, cz[AWEFD_RES_MAXNOP], cx[AWEFD_RES_MAXNOP];
+    float bz[AWEFD_RES_MAXNOP], bx[AWEFD_RES_MAXNOP];
+    const float *vel, *rho;
+    const float *sp1, *sp2;
+    float *P, *C;                /* previous and current field after the loop  */
+    int nt;
+    /* source entries per wave of each block (every node it computes) */
+    const int *ibeg;
+    const awefd_inj *inj;
+    const float *wav;
+    long wstride;
+    int wexpl;
+    /* receivers per block, by the block of their first corner */
+    int nr;
+    const int *rbeg, *ridx;
+    const int *rj;
+    const float *rw;
+    float *tr;                   /* traces, nt x nr                            */
+    /* rim words (two parities of ntz ntx rims), tag of step 0, and the flag a
+     * block raises when it gives up waiting */
+    unsigned long long *E;
+    unsigned tag0;
+    unsigned *stop;
+    /* a wait looks at the clock every wmask + 1 polls and ends after wticks of
+     * the 100 MHz wall clock */
+    unsigned wmask;
+    long long wticks;
+} awefd_res_args;
+
+/* one shot (many NULL) or the shots of a block table, all steps, cooperative
+ * (res_nop1.hip ... res_nop4.hip); resident blocks per CU (0: not compiled) */
+int awefd__res_launch1(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
+                       int vd, void *stream);
+int awefd__res_launch2(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
+                       int vd, void *stream);
+int awefd__res_launch3(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
+                       int vd, void *stream);
+int awefd__res_launch4(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
+                       int vd, void *stream);
+int awefd__res_blocks1(int rx, int S, int vd);
+int awefd__res_blocks2(int rx, int S, int vd);
+int awefd__res_blocks3(int rx, int S, int vd);
+int awefd__res_blocks4(int rx, int S, int vd);
+
 /* Adjoint of the cartesian 2-D loop (adj_kernels.hip). */
 #define AWEFD_ADJ_NWAVE 4        /* waves per block of the adjoint step kernel   */
 #ifndef AWEFD_ADJ_RX

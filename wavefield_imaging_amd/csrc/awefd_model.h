@@ -8,6 +8,22 @@
 #include "awefd.h"
 #include "awefd_internal.h"
 
+/* device memory that grows as needed */
+typedef struct {
+    void *p;
+    size_t cap;
+} awefd_res_buf;
+
+/* resident 2-D loop (awefd_resident.c): its tile, rim words, point tables */
+typedef struct {
+    int on;
+    awefd_res_tile t;
+    awefd_res_buf E, src, rec;
+    size_t inj_off, idx_off;
+    unsigned tag;                 /* next unused step tag                    */
+    unsigned *stop;               /* host memory: a block gave up waiting    */
+} awefd_res;
+
 struct awefd_model {
     awefd_params p;
     int ndim;
@@ -95,6 +111,8 @@ struct awefd_model {
     float *eager_dtr;             /* loop is captured when a run repeats it   */
     int eager_seen;
 
+    awefd_res res;
+
     /* gradient state (awefd_adjoint.c): checkpoints of the last
      * awefd_run_ckpt, valid while gen is unchanged; setters bump gen */
     void *adj;
@@ -108,6 +126,23 @@ void awefd__cart_args(const awefd_model *m, awefd_cart_args *a);
 int  awefd__ensure_traces(awefd_model *m);
 int  awefd__cart_buckets(const awefd_model *m, int tz, int ntz, int tx, awefd_inj **inj, int **ibeg,
                          int *nbucket, long *ninj);
+
+/* resident 2-D loop (awefd_resident.c) */
+int  awefd__res_form(const awefd_model *m);
+void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t);
+int  awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *one, const awefd_res_args *many,
+                       const int *bshot, int nblk, int vd, hipStream_t s);
+int  awefd__res_blocks(int nop, const awefd_res_tile *t, int vd);
+int  awefd__res_create(awefd_model *m);
+void awefd__res_free(awefd_model *m);
+int  awefd__res_set_sources(awefd_model *m);
+int  awefd__res_set_receivers(awefd_model *m);
+int  awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *out, size_t *inj_off);
+int  awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *out, size_t *idx_off);
+int  awefd__res_tags(awefd_res_buf *E, unsigned *tag, int nt, hipStream_t s, unsigned *tag0);
+void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_res_buf *src, size_t inj_off,
+                     const awefd_res_buf *rec, size_t idx_off, float *dtr, awefd_res_args *a);
+int  awefd__res_run(awefd_model *m, float *dtr, int *done);
 
 /* gradient internals shared with the batched path (awefd_adjoint.c) */
 void   awefd__adjoint_free(awefd_model *m);
