@@ -11,6 +11,7 @@
 #include <hip/hip_runtime_api.h>
 #include <math.h>
 #include <stdarg.h>
+#include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -319,6 +320,54 @@ int awefd_padded_dims(const awefd_model *m, int dims[3], int *nb)
 
 int awefd_device(const awefd_model *m) { return m ? m->dev : -1; }
 
+/* Rows between dense host memory and device rows of dpitch bytes.  A 2-D copy
+ * of pageable memory goes row by row (7 us each: 3.2 ms for the 467 rows of a
+ * 271 x 467 field, 9 ms for its velocity and density records), so the rows
+ * pass through a staging buffer of whole device rows, ROWS_STAGE bytes at a
+ * time, each piece one copy (0.1 and 0.7 ms).  Bytes beyond a row are written
+ * as zero on the way up. */
+#define ROWS_STAGE ((size_t)16 << 20)
+
+static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, size_t nrows, int up)
+{
+    if (!nrows || !row) return hipSuccess;
+    if (dpitch == row)
+        return hipMemcpy(up ? dev : host, up ? host : dev, row * nrows, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
+    size_t per = ROWS_STAGE / dpitch;
+    if (per < 1) per = 1;
+    if (per > nrows) per = nrows;
+    char *st = malloc(per * dpitch);
+    if (!st)                             /* no staging: the copy of single rows */
+        return up ? hipMemcpy2D(dev, dpitch, host, row, row, nrows, hipMemcpyHostToDevice)
+                  : hipMemcpy2D(host, row, dev, dpitch, row, nrows, hipMemcpyDeviceToHost);
+    hipError_t e = hipSuccess;
+    for (size_t r0 = 0; r0 < nrows && e == hipSuccess; r0 += per) {
+        const size_t n = nrows - r0 < per ? nrows - r0 : per;
+        if (up) {
+            for (size_t r = 0; r < n; r++) {
+                memcpy(st + r * dpitch, host + (r0 + r) * row, row);
+                memset(st + r * dpitch + row, 0, dpitch - row);
+            }
+            e = hipMemcpy(dev + r0 * dpitch, st, n * dpitch, hipMemcpyHostToDevice);
+        } else {
+            e = hipMemcpy(st, dev + r0 * dpitch, n * dpitch, hipMemcpyDeviceToHost);
+            for (size_t r = 0; e == hipSuccess && r < n; r++) memcpy(host + (r0 + r) * row, st + r * dpitch, row);
+        }
+    }
+    free(st);
+    return e;
+}
+
+hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows)
+{
+    return rows_copy(dev, dpitch, (char *)(uintptr_t)host, row, nrows, 1);
+}
+
+hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows)
+{
+    return rows_copy((char *)(uintptr_t)dev, dpitch, host, row, nrows, 0);
+}
+
 static int upload(awefd_model *m, void **dst, const void *src, size_t bytes)
 {
     free_dev(dst);
@@ -367,8 +416,7 @@ static int cart_set_density(awefd_model *m, const float *den)
     free_dev((void **)&m->drho);
     hipError_t e = hipMalloc((void **)&m->drho, sizeof(float) * 4 * (size_t)m->nalloc);
     if (e == hipSuccess)
-        e = hipMemcpy2D(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, sizeof(float) * 4 * n1,
-                        (size_t)n2 * n3, hipMemcpyHostToDevice);
+        e = awefd__rows_up(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, (size_t)n2 * n3);
     free(g);
     if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "density upload: %s", hipGetErrorString(e));
     return AWEFD_OK;
@@ -456,8 +504,7 @@ static int cart_set_model(awefd_model *m, const float *vel, const float *den)
         for (long c = 0; c < (long)n2 * n3; c++)
             for (int iz = 0; iz <= m->nb && iz < n1; iz++) v[c * n1 + iz] = 0.f;
     if (rc == 0) {
-        hipError_t e = hipMemcpy2D(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1,
-                                   sizeof(float) * n1, (size_t)n2 * n3, hipMemcpyHostToDevice);
+        hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1, (size_t)n2 * n3);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "vel upload: %s", hipGetErrorString(e));
     }
     free(v);
@@ -495,7 +542,11 @@ int awefd_set_model_dev(awefd_model *m, const float *d_vel)
                                          "velocity on the host; use awefd_set_model",
                            m->hyb ? "hybridbc=y" : "3-D dabc=y");
     HIPCHK(hipSetDevice(m->dev));
-    int rc = m->sponge ? cart_sponge_tables(m) : AWEFD_OK;
+    /* the sponge tables depend on the grid alone: made once */
+    const int tables = m->sponge && !m->dsp[2];
+    const int moved = tables || m->drho || m->p.adj;   /* adj=y: a new reversed wavelet */
+    const unsigned bgen = m->bgen;
+    int rc = tables ? cart_sponge_tables(m) : AWEFD_OK;
     if (!rc) {
         const float dt = m->p.dt;
         const int nbs[3] = {m->nb, m->nb, m->ndim == 3 ? m->nb : 0};
@@ -509,6 +560,7 @@ int awefd_set_model_dev(awefd_model *m, const float *d_vel)
         m->model_set = 1;
     }
     const int rd = setter_done(m);
+    if (!moved) m->bgen = bgen;
     return rc ? rc : rd;
 }
 
@@ -805,8 +857,7 @@ static int prof_collect(awefd_model *m, int npairs)
 /* Device field (row stride ld) to a dense host array (row stride np[0]). */
 static hipError_t copy_field_out(const awefd_model *m, float *host, const float *dev)
 {
-    return hipMemcpy2D(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld,
-                       sizeof(float) * m->np[0], (size_t)m->np[1] * m->np[2], hipMemcpyDeviceToHost);
+    return awefd__rows_down(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2]);
 }
 
 /* Apply the pending sponge factor to a host copy of the stored field (the
@@ -929,6 +980,7 @@ static int build_wrev(awefd_model *m)
 static int setter_done(awefd_model *m)
 {
     m->gen++;
+    m->bgen++;
     if (is_cart(m) && m->p.adj && m->model_set && m->src_set && m->rec_set && m->wav_set) return build_wrev(m);
     return AWEFD_OK;
 }

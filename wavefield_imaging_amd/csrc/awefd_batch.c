@@ -106,9 +106,8 @@ struct awefd_batch {
     int fwd_ok, bwd_ok;
     int fwd_depth, bwd_depth;        /* steps per pass the graphs were made for  */
     int bwd_adepth;                  /* ... and adjoint steps per pass           */
-    float *bwd_gout;
-    unsigned *mgen;                  /* each model's generation when the tables
-                                        were built (setters bump it)           */
+    unsigned *mgen;                  /* each model's buffer generation (bgen) when
+                                        the tables were built                  */
     int built;                       /* tables built for the current tile       */
 };
 
@@ -342,7 +341,7 @@ static int batch_build(awefd_batch *b, int rx, int group_mb)
         b->ngroup = ng;
         b->rx = rx;
         b->group_mb = group_mb;
-        for (int s = 0; s < b->nshot; s++) b->mgen[s] = b->m[s]->gen;
+        for (int s = 0; s < b->nshot; s++) b->mgen[s] = b->m[s]->bgen;
         b->built = 1;
     } else {
         b->built = 0;
@@ -361,7 +360,7 @@ static int batch_build(awefd_batch *b, int rx, int group_mb)
 /* The tables and the captured graphs hold each model's device pointers
  * (sponge tables, (v dt)^2, wavelet, points, trace buffer).  A setter that
  * ran on a model since they were built may have replaced those buffers (its
- * generation moved): check the shots again and rebuild everything for the
+ * buffer generation moved): check the shots again and rebuild everything for the
  * current tile before the next launch. */
 static int shots_ready(awefd_batch *b)
 {
@@ -377,7 +376,7 @@ static int batch_sync(awefd_batch *b)
 {
     int stale = !b->built, rc;
     if ((rc = shots_ready(b))) return rc;
-    for (int s = 0; s < b->nshot; s++) stale |= b->mgen[s] != b->m[s]->gen;
+    for (int s = 0; s < b->nshot; s++) stale |= b->mgen[s] != b->m[s]->bgen;
     if (!stale) return AWEFD_OK;
     const int depth = b->depth;
     if ((rc = batch_build(b, b->rx ? b->rx : 8, b->group_mb))) return rc;
@@ -1283,10 +1282,10 @@ static int adj_tables(awefd_batch *b, const float *const *d_res)
  * steps per pass at depth 3, while the pass's last field is one the segment
  * keeps, then single steps) and walked back by the adjoint steps (in pairs
  * n, n-1 inside the segment at adepth 2, a single step for an odd one
- * left); last the shots' dJ/dV summed in shot order into d_grad. */
-static int capture_bwd(awefd_batch *b, float *d_grad, int depth, int adepth)
+ * left). */
+static int capture_bwd(awefd_batch *b, int depth, int adepth)
 {
-    if (b->xbwd && b->bwd_ok && b->bwd_gout == d_grad && b->bwd_depth == depth && b->bwd_adepth == adepth)
+    if (b->xbwd && b->bwd_ok && b->bwd_depth == depth && b->bwd_adepth == adepth)
         return AWEFD_OK;
     if (b->xbwd) hipGraphExecDestroy(b->xbwd);
     if (b->gbwd) hipGraphDestroy(b->gbwd);
@@ -1314,7 +1313,6 @@ static int capture_bwd(awefd_batch *b, float *d_grad, int depth, int adepth)
                 e = awefd_launch_adj2d_batch(b->d_adj, b->d_abshot + b->agoff[g], b->agnblk[g], na, b->nop,
                                              b->stream);
         }
-    if (!e) e = awefd_launch_adj2d_chain(&b->ha[0], b->d_adj, b->nshot, d_grad, b->stream);
     if (e) rc = awefd__fail(AWEFD_EHIP, "batched backward pass: %s", hipGetErrorString((hipError_t)e));
     hipGraph_t gr = NULL;
     hipError_t he = hipStreamEndCapture(b->stream, &gr);
@@ -1326,7 +1324,6 @@ static int capture_bwd(awefd_batch *b, float *d_grad, int depth, int adepth)
     b->gbwd = gr;
     HIPCHK(hipGraphInstantiate(&b->xbwd, gr, NULL, NULL, 0));
     b->bwd_ok = 1;
-    b->bwd_gout = d_grad;
     b->bwd_depth = depth;
     b->bwd_adepth = adepth;
     return AWEFD_OK;
@@ -1352,8 +1349,11 @@ int awefd_batch_adjoint_grad(awefd_batch *b, const float *const *d_res, float *d
     /* the tables hold the residual pointers and the buffers just prepared;
      * the captured graph reads them when it runs */
     if ((rc = adj_tables(b, d_res))) return rc;
-    if ((rc = capture_bwd(b, d_grad, ckpt_depth(b), adj_depth()))) return rc;
+    if ((rc = capture_bwd(b, ckpt_depth(b), adj_depth()))) return rc;
     HIPCHK(hipGraphLaunch(b->xbwd, b->stream));
+    /* the shots' dJ/dV summed in shot order: the graph holds no output address */
+    const int e = awefd_launch_adj2d_chain(&b->ha[0], b->d_adj, b->nshot, d_grad, b->stream);
+    if (e) return awefd__fail(AWEFD_EHIP, "gradient chain: %s", hipGetErrorString((hipError_t)e));
     HIPCHK(hipStreamSynchronize(b->stream));
     return AWEFD_OK;
 }

@@ -117,6 +117,10 @@ struct awefd_model {
      * awefd_run_ckpt, valid while gen is unchanged; setters bump gen */
     void *adj;
     unsigned gen;
+    /* generation of the device buffers and points: moves when a setter may
+     * have replaced one (captured graphs and point tables refer to them), not
+     * when awefd_set_model_dev only writes new velocities */
+    unsigned bgen;
 };
 
 int awefd__fail(int code, const char *fmt, ...);
@@ -124,6 +128,8 @@ int awefd__fail(int code, const char *fmt, ...);
 /* cartesian helpers shared with the batched path (awefd_api.c) */
 void awefd__cart_args(const awefd_model *m, awefd_cart_args *a);
 int  awefd__ensure_traces(awefd_model *m);
+hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows);
+hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows);
 int  awefd__cart_buckets(const awefd_model *m, int tz, int ntz, int tx, awefd_inj **inj, int **ibeg,
                          int *nbucket, long *ninj);
 

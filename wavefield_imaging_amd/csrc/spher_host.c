@@ -260,8 +260,7 @@ int awefd__spher_set_model(awefd_model *m, const float *vel)
     awefd_pad(vel, vp, m->p.n, nbs);
     const float dt = m->p.dt;
     for (long i = 0; i < nc; i++) vv[i] = (dt * dt) * (vp[i] * vp[i]);
-    hipError_t e = hipMemcpy2D(m->dvel, sizeof(float) * m->ld, vv, sizeof(float) * n1, sizeof(float) * n1,
-                               (size_t)n2 * n3, hipMemcpyHostToDevice);
+    hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, vv, sizeof(float) * n1, (size_t)n2 * n3);
     free(vv);
     if (e != hipSuccess) {
         free(vp);
@@ -567,8 +566,8 @@ int awefd__spher_loop(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
             }
             hipError_t he = hipStreamSynchronize(m->stream);
             if (he == hipSuccess)
-                he = hipMemcpy2D(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld,
-                                 sizeof(float) * m->np[0], (size_t)m->np[1] * m->np[2], hipMemcpyDeviceToHost);
+                he = awefd__rows_down(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld,
+                                      (size_t)m->np[1] * m->np[2]);
             if (he != hipSuccess) {
                 rc = awefd__fail(AWEFD_EHIP, "snapshot copy: %s", hipGetErrorString(he));
                 break;
@@ -594,7 +593,6 @@ int awefd__spher_loop(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
 int awefd__spher_get_field(awefd_model *m, float *host)
 {
     HIPCHK(hipStreamSynchronize(m->stream));
-    HIPCHK(hipMemcpy2D(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld, sizeof(float) * m->np[0],
-                       (size_t)m->np[1] * m->np[2], hipMemcpyDeviceToHost));
+    HIPCHK(awefd__rows_down(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2]));
     return AWEFD_OK;
 }
