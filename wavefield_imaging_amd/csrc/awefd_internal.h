@@ -349,7 +349,16 @@ typedef struct {
     const int *rj;           /* (jr, jtheta, jphi) per receiver               */
     const float *rw;
     float *trow;
+    /* fused extraction and next injection: the box (r, theta, phi; low, high)
+     * of the injection nodes, and the receivers with a corner in it */
+    int box[6];
+    int nconf;
+    const int *conf;
 } awefd_spher_args;
+
+/* injection nodes and boxed receivers the fused launch's first block takes */
+#define AWEFD_SPHER_FUSE_NODES 256
+#define AWEFD_SPHER_FUSE_CONF 1024
 
 /* Launchers (cart_kernels.hip).  Return 0 or a HIP error code. */
 int awefd_launch_cart_step(const awefd_cart_args *a, int nop, int ndim, int sse, int varden,
@@ -397,6 +406,9 @@ int awefd_launch_spher_inject(const awefd_spher_args *a, void *stream);
 int awefd_launch_spher_step(const awefd_spher_args *a, void *stream);
 int awefd_launch_spher_shell(const awefd_spher_args *a, void *stream);
 int awefd_launch_spher_extract(const awefd_spher_args *a, void *stream);
+/* extraction of step it and injection of step it + 1 into the field just
+ * finished (Q) */
+int awefd_launch_spher_points(const awefd_spher_args *a, void *stream);
 int awefd_spher_step_occupancy(int ndim);
 
 #ifdef __cplusplus

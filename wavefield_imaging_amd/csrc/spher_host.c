@@ -42,6 +42,8 @@ typedef struct {
     int ninode;
     int inj_dirty;
     int *d_rrtp;                     /* receiver map in (r, theta, phi) order     */
+    int box[6], nconf;               /* box of the injection nodes, the receivers */
+    int *d_conf;                     /* with a corner in it                       */
     float *h_velp;                   /* padded raw velocity                       */
     unsigned nsr, nst, nsp;
     float tdr, dr2, tdt, dt2, dp2;
@@ -51,6 +53,7 @@ typedef struct {
 
 static spher_state *st(awefd_model *m) { return (spher_state *)m->spher; }
 static int build_injection(awefd_model *m);
+static int build_conflicts(awefd_model *m);
 
 static void dfree(void *pp)
 {
@@ -84,6 +87,7 @@ void awefd__spher_free(awefd_model *m)
     dfree(&s->d_ibeg);
     dfree(&s->d_iw);
     dfree(&s->d_rrtp);
+    dfree(&s->d_conf);
     free(s->h_velp);
     free(s);
     m->spher = NULL;
@@ -112,10 +116,16 @@ static void spher_tiling(awefd_model *m)
     if (m->col) {
         /* columns of 64 r x AWEFD_SPHER_CRX theta, phi chunks of about
          * AWEFD_SPHER_CHUNK planes (default 12: 0.563 ms per step on the
-         * 460 x 572 x 572 shell; 6-8 planes 0.577, 16 0.567); blocks: 8 XCD
-         * shares of ceil(ntx / 8) theta tiles */
+         * 460 x 572 x 572 shell; 6-8 planes 0.577, 16 0.567), down to 4 where
+         * 12 would leave the chip short of the 6 waves per SIMD it holds (one
+         * wave's chunk then bounds the step: 114 x 142 x 142, 12 planes
+         * 22.8 us, 8 19.2, 6 17.5, 4 15.3, 3 16, 2 17); blocks: 8 XCD shares of
+         * ceil(ntx / 8) theta tiles */
         const char *ch = getenv("AWEFD_SPHER_CHUNK");
-        const long chunk = ch && atol(ch) > 0 ? atol(ch) : 12;
+        int cus = 256;
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev);
+        const long full = (long)m->ntz * ((n2 + AWEFD_SPHER_CRX - 1) / AWEFD_SPHER_CRX) * n3 / (24L * cus);
+        const long chunk = ch && atol(ch) > 0 ? atol(ch) : full < 4 ? 4 : full < 12 ? full : 12;
         m->ntx = (n2 + AWEFD_SPHER_CRX - 1) / AWEFD_SPHER_CRX;
         long nty = (n3 + chunk - 1) / chunk;
         m->nty = (int)(nty < 1 ? 1 : nty > n3 ? n3 : nty);
@@ -349,6 +359,38 @@ int awefd__spher_set_receivers(awefd_model *m)
     }
     int rc = up(&s->d_rrtp, h, sizeof(int) * 3 * (m->nr > 0 ? m->nr : 1));
     free(h);
+    return rc ? rc : s->inj_dirty || !m->h_sj ? AWEFD_OK : build_conflicts(m);
+}
+
+/* The box of the injection nodes and the receivers that read a node of it
+ * (the extraction has to read them before the next injection); built by
+ * whichever of the point setters comes last. */
+static int build_conflicts(awefd_model *m)
+{
+    spher_state *s = st(m);
+    const int ax[3] = {1, 0, 2};                   /* (r, theta, phi) of the point map */
+    for (int k = 0; k < 3; k++) {
+        s->box[2 * k] = 0x7fffffff;
+        s->box[2 * k + 1] = -1;
+        for (int i = 0; i < m->ns; i++) {
+            const int j = k < m->ndim ? m->h_sj[3 * i + ax[k]] : 0;
+            if (j < s->box[2 * k]) s->box[2 * k] = j;
+            if (j + 1 > s->box[2 * k + 1]) s->box[2 * k + 1] = j + 1;
+        }
+    }
+    s->nconf = 0;
+    int *h = malloc(sizeof(int) * (m->nr > 0 ? m->nr : 1));
+    if (!h) return awefd__fail(AWEFD_ENOMEM, "receivers near sources");
+    for (int r = 0; r < m->nr; r++) {
+        int hit = 1;
+        for (int k = 0; k < m->ndim; k++) {
+            const int j = m->h_rj[3 * r + ax[k]];
+            hit = hit && j + 1 >= s->box[2 * k] && j <= s->box[2 * k + 1];
+        }
+        if (hit) h[s->nconf++] = r;
+    }
+    const int rc = up(&s->d_conf, h, sizeof(int) * s->nconf);
+    free(h);
     return rc;
 }
 
@@ -452,7 +494,7 @@ static int build_injection(awefd_model *m)
     }
     free(e); free(node); free(ibeg); free(iw);
     if (!rc) s->inj_dirty = 0;
-    return rc;
+    return rc || !m->h_rj ? rc : build_conflicts(m);
 }
 
 static void spher_args(const awefd_model *m, awefd_spher_args *a)
@@ -515,6 +557,9 @@ static void spher_args(const awefd_model *m, awefd_spher_args *a)
     a->nr = m->nr;
     a->rj = m->d_rj;
     a->rw = m->d_rw;
+    memcpy(a->box, s->box, sizeof a->box);
+    a->nconf = s->nconf;
+    a->conf = s->d_conf;
 }
 
 /* The time loop (MAWEFDspher2Dcpu.c:264-317, MAWEFDspher3Dcpu.c:302-359).
@@ -538,18 +583,23 @@ int awefd__spher_loop(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
         for (int i = m->nev; i < 2 * nt; i++) hipEventCreate(&m->ev[i]);
         m->nev = 2 * nt;
     }
+    /* extraction and the next injection in one launch (k_spher_points), unless
+     * a snapshot shows the field between them */
+    const int fuse = !(cb && jsnap > 0) && a.ninode > 0 && a.ninode <= AWEFD_SPHER_FUSE_NODES &&
+                     a.nconf <= AWEFD_SPHER_FUSE_CONF;
     for (int it = 0; it < nt && !rc; it++) {
         a.P = m->dC;
         a.Q = m->dP;
         a.it = it;
         a.trow = dtr ? dtr + (long)it * m->nr : m->d_traces + (long)it * m->nr;
-        int e = awefd_launch_spher_inject(&a, m->stream);
+        int e = fuse && it > 0 ? 0 : awefd_launch_spher_inject(&a, m->stream);
         if (m->prof) hipEventRecord(m->ev[2 * npairs], m->stream);
         if (!e) e = awefd_launch_spher_step(&a, m->stream);
         if (m->prof) hipEventRecord(m->ev[2 * npairs + 1], m->stream);
         if (m->prof) npairs++;
         if (!e) e = awefd_launch_spher_shell(&a, m->stream);
-        if (!e) e = awefd_launch_spher_extract(&a, m->stream);
+        if (!e) e = fuse && it + 1 < nt ? awefd_launch_spher_points(&a, m->stream)
+                                        : awefd_launch_spher_extract(&a, m->stream);
         if (e) {
             rc = awefd__fail(AWEFD_EHIP, "step %d launch: %s", it, hipGetErrorString((hipError_t)e));
             break;

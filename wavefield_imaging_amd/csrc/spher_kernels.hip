@@ -156,51 +156,63 @@ __device__ __forceinline__ long offs(const awefd_spher_args &a, node3 c)
  * node's last rule; uo(n) is n's pre-boundary value S(n) for a low-face rule
  * and n's final value for a high-face rule.  The chain of high-face rules is
  * walked inward to its end, then evaluated outward in the reference's order.
- * This form walks the chain again for every level; shell_final below keeps
- * the levels in registers and falls back to it for chains deeper than that. */
-template <int NDIM>
-__device__ __forceinline__ float shell_final_walk(const awefd_spher_args &a, node3 c0)
+ *
+ * The first CHAIN_REG levels stay in registers: level l holds the current
+ * field at chain node c_l, at its inward neighbour c_(l+1) and the one-way
+ * coefficient of c_l's rule, all loaded on the way in (no load waits for
+ * another), then x = P(c_(l+1)) + (P(c_l) - x) b_l outward from the chain's
+ * end.  On the 460 x 572 x 572 shell 99.8 % of the nodes have at most 2
+ * levels (6.66 M none, 1.67 M one, 1.67 M two, 20 K up to 8).  A deeper chain
+ * is walked again from its start, without loads, the rules packed 3 bits
+ * each, and evaluated on the way back: walked once more for every level, the
+ * few waves that hold such a chain took as long as the rest of the pass on a
+ * 114 x 142 x 142 shell (21.0 us a launch, now 13.4; on the large shell, whose
+ * other waves hid them, 97 and 95).  With the loads of 2 or 4 levels in flight
+ * 13.0 and 12.9 us, but 67-70 VGPRs, a wave per SIMD less: the large shell
+ * 100 us. */
+constexpr int CHAIN_REG = 2;
+static_assert(3 * AWEFD_SPHER_MAXCHAIN <= 64, "packed rules");
+
+__device__ __forceinline__ bool high_rule(int r) { return r == 2 || r == 4 || r == 6; }
+
+/* the chain node whose inward neighbour by a high rule is c */
+__device__ __forceinline__ node3 outward(node3 c, int rule)
 {
-    const int n1 = a.n1, n2 = a.n2, n3 = a.n3;
-    int rule = oneway_rule<NDIM>(c0.r, c0.t, c0.p, n1, n2, n3);
-    node3 c = c0;
-    int depth = 0;
-    while ((rule == 2 || rule == 4 || rule == 6) && depth < AWEFD_SPHER_MAXCHAIN) {
+    if (rule == 2) c.t++;
+    else if (rule == 4) c.r++;
+    else c.p++;
+    return c;
+}
+
+/* one-way value of node c by a low rule, its own field pc given */
+__device__ __forceinline__ float low_end(const awefd_spher_args &a, node3 c, int rule, float pc)
+{
+    const node3 n = inward(c, rule);
+    return a.P[offs(a, n)] + (pc - a.S[offs(a, n)]) * oneway_coef(a, c, rule);
+}
+
+/* the final value of a node whose chain is deeper than the registers hold */
+template <int NDIM>
+__device__ __forceinline__ float deep_chain(const awefd_spher_args &a, node3 c)
+{
+    unsigned long long rs = 0;
+    int n = 0, rule = oneway_rule<NDIM>(c.r, c.t, c.p, a.n1, a.n2, a.n3);
+    while (high_rule(rule) && n < AWEFD_SPHER_MAXCHAIN) {
+        rs |= (unsigned long long)rule << (3 * n++);
         c = inward(c, rule);
-        rule = oneway_rule<NDIM>(c.r, c.t, c.p, n1, n2, n3);
-        depth++;
+        rule = oneway_rule<NDIM>(c.r, c.t, c.p, a.n1, a.n2, a.n3);
     }
-    float x;
-    if (rule == 0) {
-        x = a.S[offs(a, c)];
-    } else {
-        const node3 n = inward(c, rule);
-        x = a.P[offs(a, n)] + (a.P[offs(a, c)] - a.S[offs(a, n)]) * oneway_coef(a, c, rule);
-    }
-    for (int l = depth - 1; l >= 0; l--) {
-        node3 cl = c0;
-        int rl = oneway_rule<NDIM>(cl.r, cl.t, cl.p, n1, n2, n3);
-        for (int m = 0; m < l; m++) {
-            cl = inward(cl, rl);
-            rl = oneway_rule<NDIM>(cl.r, cl.t, cl.p, n1, n2, n3);
-        }
-        const node3 n = inward(cl, rl);
-        x = a.P[offs(a, n)] + (a.P[offs(a, cl)] - x) * oneway_coef(a, cl, rl);
+    float pn = a.P[offs(a, c)];
+    float x = rule == 0 ? a.S[offs(a, c)] : low_end(a, c, rule, pn);
+    for (int l = n - 1; l >= 0; l--) {
+        const int r = (int)(rs >> (3 * l)) & 7;
+        c = outward(c, r);
+        const float pl = a.P[offs(a, c)];
+        x = pn + (pl - x) * oneway_coef(a, c, r);
+        pn = pl;
     }
     return x;
 }
-
-/* The same value, the chain's levels kept in registers: level l holds the
- * current field at chain node c_l, at its inward neighbour c_(l+1) and the
- * one-way coefficient of c_l's rule, all loaded on the way in (no load waits
- * for another), then x = P(c_(l+1)) + (P(c_l) - x) b_l outward from the
- * chain's end, the same operations in the same order.  Chains are at most 8
- * deep, and on the 460 x 572 x 572 shell 99.8 % of the nodes have at most
- * 2 levels (6.66 M none, 1.67 M one, 1.67 M two, 20 K deeper); a deeper
- * chain takes the walk above. */
-constexpr int CHAIN_REG = 2;
-
-__device__ __forceinline__ bool high_rule(int r) { return r == 2 || r == 4 || r == 6; }
 
 template <int NDIM>
 __device__ __forceinline__ float shell_final(const awefd_spher_args &a, node3 c0)
@@ -223,14 +235,8 @@ __device__ __forceinline__ float shell_final(const awefd_spher_args &a, node3 c0
         rule = oneway_rule<NDIM>(c.r, c.t, c.p, n1, n2, n3);
         depth = l + 1;
     }
-    if (high_rule(rule)) return shell_final_walk<NDIM>(a, c0);
-    float x;
-    if (rule == 0) {
-        x = a.S[offs(a, c)];
-    } else {
-        const node3 n = inward(c, rule);
-        x = a.P[offs(a, n)] + (pcur - a.S[offs(a, n)]) * oneway_coef(a, c, rule);
-    }
+    if (high_rule(rule)) return deep_chain<NDIM>(a, c0);
+    float x = rule == 0 ? a.S[offs(a, c)] : low_end(a, c, rule, pcur);
 #pragma unroll
     for (int l = CHAIN_REG - 1; l >= 0; l--)
         if (l < depth) x = pn[l] + (pc[l] - x) * bc[l];
@@ -306,11 +312,10 @@ __global__ __launch_bounds__(256) void k_spher_shell(const awefd_spher_args a)
     shell_node<NDIM>(a, blockIdx.x * 256u + threadIdx.x);
 }
 
-/* Injection of step it into field F at injection node i; a node's
- * contributions are added in the reference's source order. */
-__device__ __forceinline__ void inject_node(const awefd_spher_args &a, float *F, int it, int i)
+/* Value of injection node i (offset o) of field F after the injection of
+ * step it; a node's contributions are added in the reference's source order. */
+__device__ __forceinline__ float injected(const awefd_spher_args &a, const float *F, int it, int i, long o)
 {
-    const long o = a.inode[i];
     const float wa = a.wav[it];
     float v = F[o];
     for (int e = a.ibeg[i]; e < a.ibeg[i + 1]; e++) {
@@ -318,7 +323,7 @@ __device__ __forceinline__ void inject_node(const awefd_spher_args &a, float *F,
         inc = inc * a.iw[2 * e + 1];   /* reflectivity (1 for constant injection) */
         v = v + inc;
     }
-    F[o] = v;
+    return v;
 }
 
 /* Injection into the current field before the solve, one thread per node. */
@@ -326,15 +331,14 @@ __global__ __launch_bounds__(256) void k_spher_inject(const awefd_spher_args a)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= a.ninode) return;
-    inject_node(a, a.P, a.it, i);
+    const long o = a.inode[i];
+    a.P[o] = injected(a, a.P, a.it, i, o);
 }
 
-/* Receiver gather from the finished field of the step. */
+/* Receiver r's value of the finished field of the step. */
 template <int NDIM>
-__global__ __launch_bounds__(256) void k_spher_extract(const awefd_spher_args a)
+__device__ __forceinline__ void extract_node(const awefd_spher_args &a, int r)
 {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= a.nr) return;
     const long sy = (long)a.ld * a.n2;
     const long b = (long)a.rj[3 * r + 2] * sy + (long)a.rj[3 * r + 1] * a.ld + a.rj[3 * r];
     constexpr int NC = NDIM == 3 ? 8 : 4;
@@ -346,6 +350,45 @@ __global__ __launch_bounds__(256) void k_spher_extract(const awefd_spher_args a)
         s = q == 0 ? term : s + term;
     }
     a.trow[r] = s;
+}
+
+/* Receiver gather. */
+template <int NDIM>
+__global__ __launch_bounds__(256) void k_spher_extract(const awefd_spher_args a)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r < a.nr) extract_node<NDIM>(a, r);
+}
+
+/* Receiver gather of step it and injection of step it + 1 into the same
+ * field, one launch: each is a few microseconds of launch for a few hundred
+ * nanoseconds of work (400 x 512 polar section: 2.5 + 2.5 us of a 13 us step).
+ * The receivers with a corner in the box of the injection nodes (the host
+ * lists them) are read by the first block before it injects; the others read
+ * nothing that the injection writes.  For at most AWEFD_SPHER_FUSE_NODES
+ * injection nodes and AWEFD_SPHER_FUSE_CONF such receivers: one block's
+ * share must not outlast the rest. */
+template <int NDIM>
+__global__ __launch_bounds__(256) void k_spher_points(const awefd_spher_args a)
+{
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        for (int i = tid; i < a.nconf; i += 256) extract_node<NDIM>(a, a.conf[i]);
+        const bool in = tid < a.ninode;
+        const long o = in ? a.inode[tid] : 0;
+        float v = 0.f;
+        if (in) v = injected(a, a.Q, a.it + 1, tid, o);
+        __syncthreads();
+        if (in) a.Q[o] = v;
+        return;
+    }
+    const int r = (blockIdx.x - 1) * 256 + tid;
+    if (r >= a.nr) return;
+    const int jr = a.rj[3 * r], jt = a.rj[3 * r + 1], jp = a.rj[3 * r + 2];
+    if (jr + 1 >= a.box[0] && jr <= a.box[1] && jt + 1 >= a.box[2] && jt <= a.box[3] &&
+        (NDIM == 2 || (jp + 1 >= a.box[4] && jp <= a.box[5])))
+        return;
+    extract_node<NDIM>(a, r);
 }
 
 /* x / c for a launch divisor c.  FD: (float)((double)x * rc) with rc = 1/c in
@@ -752,6 +795,15 @@ extern "C" int awefd_launch_spher_extract(const awefd_spher_args *a, void *strea
     const dim3 g((a->nr + 255) / 256);
     if (a->ndim == 3) hipLaunchKernelGGL(k_spher_extract<3>, g, dim3(256), 0, (hipStream_t)stream, *a);
     else hipLaunchKernelGGL(k_spher_extract<2>, g, dim3(256), 0, (hipStream_t)stream, *a);
+    return (int)hipGetLastError();
+}
+
+extern "C" int awefd_launch_spher_points(const awefd_spher_args *a, void *stream)
+{
+    if (a->ninode > AWEFD_SPHER_FUSE_NODES) return (int)hipErrorInvalidValue;
+    const dim3 g(1 + (a->nr + 255) / 256);
+    if (a->ndim == 3) hipLaunchKernelGGL(k_spher_points<3>, g, dim3(256), 0, (hipStream_t)stream, *a);
+    else hipLaunchKernelGGL(k_spher_points<2>, g, dim3(256), 0, (hipStream_t)stream, *a);
     return (int)hipGetLastError();
 }
 
