@@ -1116,12 +1116,13 @@ static int run_common(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
     if (rc) return rc;
     HIPCHK(hipSetDevice(m->dev));
     if ((rc = awefd__ensure_traces(m))) return rc;
-    const int plain2d = is_cart(m) && m->ndim == 2 && !m->prof && !(cb && jsnap > 0);
+    const int whole2d = m->ndim == 2 && !m->prof && !(cb && jsnap > 0), plain2d = whole2d && is_cart(m);
     float *trow0 = dtr ? dtr : m->d_traces;
-    if (plain2d && m->res.on) {
-        /* the resident loop starts from zero fields of its own */
+    if (whole2d && m->res.on) {
+        /* the resident loops start from zero fields of their own */
         int done;
-        if ((rc = awefd__res_run(m, trow0, &done)) || done) return rc;
+        rc = is_cart(m) ? awefd__res_run(m, trow0, &done) : awefd__polar_run(m, trow0, &done);
+        if (rc || done) return rc;
     }
     if ((rc = awefd_reset(m))) return rc;
     const int repeat = plain2d && ((m->cvalid && m->cgen == m->gen && m->cdtr == trow0) ||

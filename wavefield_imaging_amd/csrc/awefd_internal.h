@@ -360,6 +360,51 @@ typedef struct {
 #define AWEFD_SPHER_FUSE_NODES 256
 #define AWEFD_SPHER_FUSE_CONF 1024
 
+/* The resident polar loop (res_polar.hip): tiles as awefd_res_tile's, with a
+ * stencil half-width of 1. */
+#define AWEFD_POLAR_ITEMS 1024   /* one-way nodes of a block (two a thread)    */
+#define AWEFD_POLAR_FACE 8       /* nodes a tile at a high face owns, at least */
+typedef struct {
+    int off, noff;               /* image offsets of the node and its inward   */
+    int nnoff;                   /* neighbour; >= 0: that one's own (its value */
+    float b, b2;                 /* is final); coefficients of the two rules   */
+    int zero;                    /* free surface                               */
+    double damp;
+} awefd_polar_item;
+typedef struct {
+    int n1, n2, ld;              /* padded r, theta, row stride                */
+    int ntz, ntx;
+    int nb, fsrf;
+    const float *pc;             /* polar coefficients, 5 per r                */
+    const float *vv;
+    const double *damp;          /* sponge table by depth                      */
+    float *P, *C;                /* previous and current field after the loop  */
+    int nt;
+    /* injection nodes of every block's image: image offset, node number */
+    const int *sbeg, *snode;
+    const int *ibeg;             /* contributions of a node, in source order   */
+    const float *iw;
+    const float *wav;
+    /* one-way nodes of every block */
+    const int *obeg;
+    const awefd_polar_item *items;
+    /* receivers per block, by the block of their first corner */
+    int nr;
+    const int *rbeg, *ridx;
+    const int *rj;               /* (jr, jtheta, jphi)                         */
+    const float *rw;
+    float *tr;
+    unsigned long long *E;
+    unsigned tag0;
+    unsigned *stop;
+    unsigned wmask;
+    long long wticks;
+} awefd_polar_args;
+/* every step of one polar grid, cooperative; resident blocks per CU (0: not
+ * compiled) */
+int awefd__polar_launch(const awefd_polar_args *a, int nblk, int rx, int S, void *stream);
+int awefd__polar_blocks(int rx, int S);
+
 /* Launchers (cart_kernels.hip).  Return 0 or a HIP error code. */
 int awefd_launch_cart_step(const awefd_cart_args *a, int nop, int ndim, int sse, int varden,
                            void *stream);

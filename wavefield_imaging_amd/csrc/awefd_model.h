@@ -18,8 +18,8 @@ typedef struct {
 typedef struct {
     int on;
     awefd_res_tile t;
-    awefd_res_buf E, src, rec;
-    size_t inj_off, idx_off;
+    awefd_res_buf E, src, rec, one;   /* one: polar one-way nodes            */
+    size_t inj_off, idx_off, one_off;
     unsigned tag;                 /* next unused step tag                    */
     unsigned *stop;               /* host memory: a block gave up waiting    */
 } awefd_res;
@@ -149,6 +149,13 @@ int  awefd__res_tags(awefd_res_buf *E, unsigned *tag, int nt, hipStream_t s, uns
 void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_res_buf *src, size_t inj_off,
                      const awefd_res_buf *rec, size_t idx_off, float *dtr, awefd_res_args *a);
 int  awefd__res_run(awefd_model *m, float *dtr, int *done);
+int  awefd__res_grow(awefd_res_buf *b, size_t bytes);
+void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_tile *t);
+int  awefd__res_buffers(awefd_model *m);
+void awefd__res_wait(unsigned *wmask, long long *wticks);
+int  awefd__res_finish(awefd_model *m, int launched, int *done);
+/* resident polar loop (spher_host.c) */
+int  awefd__polar_run(awefd_model *m, float *dtr, int *done);
 
 /* gradient internals shared with the batched path (awefd_adjoint.c) */
 void   awefd__adjoint_free(awefd_model *m);

@@ -2,7 +2,7 @@
  * Host side of the resident 2-D loop (res_loop.h): which models take it, its
  * tile, its point tables and its launches.
  *
- * A model takes it when it is cartesian 2-D in the SSE order with fdorder up
+ * A cartesian model takes it when it is 2-D in the SSE order with fdorder up
  * to 8, bilinear points, no hybrid boundary, and a compiled tile whose blocks
  * are at most the CUs.  Profiled runs, runs with snapshots and
  * awefd_run_noalloc keep the loop of one launch per step.  AWEFD_RESIDENT=0
@@ -27,7 +27,7 @@
     } while (0)
 
 /* device memory that grows and is otherwise reused */
-static int grow(awefd_res_buf *b, size_t bytes)
+int awefd__res_grow(awefd_res_buf *b, size_t bytes)
 {
     if (b->cap >= bytes && b->p) return AWEFD_OK;
     hipFree(b->p);
@@ -56,14 +56,15 @@ static launch_fn *const LAUNCH[AWEFD_RES_MAXNOP] = {awefd__res_launch1, awefd__r
 static blocks_fn *const BLOCKS[AWEFD_RES_MAXNOP] = {awefd__res_blocks1, awefd__res_blocks2, awefd__res_blocks3,
                                                     awefd__res_blocks4};
 
-/* A tile of rx rows per wave and S steps per exchange on this grid. */
-static void tile_of(const awefd_model *m, int rx, int S, awefd_res_tile *t)
+/* A tile of rx rows per wave and S steps per exchange on this grid, for a
+ * stencil half-width nop. */
+void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_tile *t)
 {
-    const int H = S * m->nop;
+    const int H = S * nop;
     t->rx = rx;
     t->S = S;
     t->zw = 64 - 2 * H;
-    t->ox = AWEFD_RES_NWAVE * rx - 2 * (S - 1) * m->nop;
+    t->ox = AWEFD_RES_NWAVE * rx - 2 * (S - 1) * nop;
     t->on = t->ox >= H;
     t->ntz = (m->np[0] + t->zw - 1) / t->zw;
     t->ntx = t->on ? (m->np[1] + t->ox - 1) / t->ox : 0;
@@ -83,7 +84,7 @@ void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t)
         const int *list = S == 1 ? (vd ? rx1 + 9 : rx1) : vd ? rx2v : rx2;
         if (e && atoi(e) != S) continue;
         for (; *list; list++) {
-            tile_of(m, *list, S, t);
+            awefd__res_tile_of(m, m->nop, *list, S, t);
             if (t->on && (long)t->ntz * t->ntx <= nblk) return;
         }
     }
@@ -101,6 +102,24 @@ int awefd__res_blocks(int nop, const awefd_res_tile *t, int vd)
     return BLOCKS[nop - 1](t->rx, t->S, vd);
 }
 
+/* rim words and the stop flag of the tile picked; on */
+int awefd__res_buffers(awefd_model *m)
+{
+    awefd_res *r = &m->res;
+    const size_t eb = sizeof(unsigned long long) * 2 * (size_t)r->t.words * r->t.ntz * r->t.ntx;
+    if (awefd__res_grow(&r->E, eb)) return AWEFD_ENOMEM;
+    const int e = awefd_launch_fill(r->E.p, (long)(eb / sizeof(float)), 0.f, m->stream);
+    if (e) return awefd__fail(AWEFD_EHIP, "resident rims: %s", hipGetErrorString((hipError_t)e));
+    HIPCHK(hipHostMalloc((void **)&r->stop, sizeof(unsigned), hipHostMallocDefault));
+    *r->stop = 0;
+    r->tag = 1;
+    r->on = 1;
+    if (getenv("AWEFD_VERBOSE"))
+        fprintf(stderr, "awefd: resident 2-D loop: %d x %d blocks, %d rows per wave, %d steps per exchange\n", r->t.ntz,
+                r->t.ntx, r->t.rx, r->t.S);
+    return AWEFD_OK;
+}
+
 int awefd__res_create(awefd_model *m)
 {
     awefd_res *r = &m->res;
@@ -114,18 +133,7 @@ int awefd__res_create(awefd_model *m)
     awefd__res_pick(m, vd, cus, &r->t);
     if (!r->t.on && vd) awefd__res_pick(m, 0, cus, &r->t);
     if (!r->t.on || awefd__res_blocks(m->nop, &r->t, 0) < 1) return AWEFD_OK;
-    const size_t eb = sizeof(unsigned long long) * 2 * (size_t)r->t.words * r->t.ntz * r->t.ntx;
-    if (grow(&r->E, eb)) return AWEFD_ENOMEM;
-    const int e = awefd_launch_fill(r->E.p, (long)(eb / sizeof(float)), 0.f, m->stream);
-    if (e) return awefd__fail(AWEFD_EHIP, "resident rims: %s", hipGetErrorString((hipError_t)e));
-    HIPCHK(hipHostMalloc((void **)&r->stop, sizeof(unsigned), hipHostMallocDefault));
-    *r->stop = 0;
-    r->tag = 1;
-    r->on = 1;
-    if (getenv("AWEFD_VERBOSE"))
-        fprintf(stderr, "awefd: resident 2-D loop: %d x %d blocks, %d rows per wave, %d steps per exchange\n", r->t.ntz,
-                r->t.ntx, r->t.rx, r->t.S);
-    return AWEFD_OK;
+    return awefd__res_buffers(m);
 }
 
 void awefd__res_free(awefd_model *m)
@@ -134,6 +142,7 @@ void awefd__res_free(awefd_model *m)
     hipFree(r->E.p);
     hipFree(r->src.p);
     hipFree(r->rec.p);
+    hipFree(r->one.p);
     if (r->stop) hipHostFree(r->stop);
     memset(r, 0, sizeof *r);
 }
@@ -178,7 +187,7 @@ int awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *o
         const size_t bytes = head + sizeof(*e) * (size_t)(beg[nb] > 0 ? beg[nb] : 1);
         for (int b = nb; b > 0; b--) beg[b] = beg[b - 1];
         beg[0] = 0;
-        rc = grow(out, bytes);
+        rc = awefd__res_grow(out, bytes);
         hipError_t he = rc ? hipSuccess : hipMemcpy(out->p, h, bytes, hipMemcpyHostToDevice);
         if (he != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident source table: %s", hipGetErrorString(he));
         *inj_off = head;
@@ -204,7 +213,7 @@ int awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf 
     for (int b = nb; b > 0; b--) h[b] = h[b - 1];
     h[0] = 0;
     const size_t bytes = sizeof(int) * ((size_t)nb + 1 + (nr > 0 ? nr : 1));
-    int rc = grow(out, bytes);
+    int rc = awefd__res_grow(out, bytes);
     if (!rc) {
         hipError_t he = hipMemcpy(out->p, h, bytes, hipMemcpyHostToDevice);
         if (he != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident receiver table: %s", hipGetErrorString(he));
@@ -238,6 +247,16 @@ int awefd__res_tags(awefd_res_buf *E, unsigned *tag, int nt, hipStream_t s, unsi
     *tag0 = *tag;
     *tag += (unsigned)nt + 1u;
     return AWEFD_OK;
+}
+
+/* 4 s; AWEFD_RES_WAIT=0 gives up at the first poll that finds a word missing
+ * (a test's way to the other loop) */
+void awefd__res_wait(unsigned *wmask, long long *wticks)
+{
+    const char *w = getenv("AWEFD_RES_WAIT");
+    const int none = w && atoi(w) == 0;
+    *wmask = none ? 0u : 1023u;
+    *wticks = none ? -1LL : 400000000LL;
 }
 
 void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_res_buf *src, size_t inj_off,
@@ -276,12 +295,27 @@ void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_
     a->rj = m->d_rj;
     a->rw = m->d_rw;
     a->tr = dtr;
-    /* 4 s; AWEFD_RES_WAIT=0 gives up at the first poll that finds a word
-     * missing (a test's way to the other loop) */
-    const char *w = getenv("AWEFD_RES_WAIT");
-    const int none = w && atoi(w) == 0;
-    a->wmask = none ? 0u : 1023u;
-    a->wticks = none ? -1LL : 400000000LL;
+    awefd__res_wait(&a->wmask, &a->wticks);
+}
+
+/* After a launch: its wait, and whether every block went through (*done). */
+int awefd__res_finish(awefd_model *m, int launched, int *done)
+{
+    awefd_res *r = &m->res;
+    if (launched) {
+        /* not launched: this device cannot hold the blocks */
+        (void)hipGetLastError();
+        r->on = 0;
+        return AWEFD_OK;
+    }
+    HIPCHK(hipStreamSynchronize(m->stream));
+    if (*(volatile unsigned *)r->stop) {
+        *r->stop = 0;
+        return AWEFD_OK;
+    }
+    m->steps_done = m->nsteps;
+    *done = 1;
+    return AWEFD_OK;
 }
 
 /* The whole loop of a set-up model; *done = 0: not taken (or given up on
@@ -299,19 +333,6 @@ int awefd__res_run(awefd_model *m, float *dtr, int *done)
     a.stop = r->stop;
     int rc = awefd__res_tags(&r->E, &r->tag, a.nt, m->stream, &a.tag0);
     if (rc) return rc;
-    const int e = awefd__res_launch(m->nop, &r->t, &a, NULL, NULL, r->t.ntz * r->t.ntx, vd, m->stream);
-    if (e) {
-        /* not launched: this device cannot hold the blocks */
-        (void)hipGetLastError();
-        r->on = 0;
-        return AWEFD_OK;
-    }
-    HIPCHK(hipStreamSynchronize(m->stream));
-    if (*(volatile unsigned *)r->stop) {
-        *r->stop = 0;
-        return AWEFD_OK;
-    }
-    m->steps_done = m->nsteps;
-    *done = 1;
-    return AWEFD_OK;
+    return awefd__res_finish(m, awefd__res_launch(m->nop, &r->t, &a, NULL, NULL, r->t.ntz * r->t.ntx, vd, m->stream),
+                             done);
 }

@@ -54,6 +54,10 @@ typedef struct {
 static spher_state *st(awefd_model *m) { return (spher_state *)m->spher; }
 static int build_injection(awefd_model *m);
 static int build_conflicts(awefd_model *m);
+static int polar_create(awefd_model *m);
+static int polar_sources(awefd_model *m, const long *node, int n);
+static int polar_receivers(awefd_model *m);
+static int polar_oneway(awefd_model *m, float *const t[4]);
 
 static void dfree(void *pp)
 {
@@ -250,7 +254,7 @@ int awefd__spher_create(awefd_model *m)
     for (int i = 0; i <= nb; i++) damp[i] = awefd_spher_damp(i, nb);
     rc = up(&m->d_damp, damp, sizeof(double) * (nb + 1));
     free(damp);
-    return rc;
+    return rc ? rc : polar_create(m);
 }
 
 /* Model: pad, (dt*dt)*(v*v), one-way tables (MAWEFDspher2Dcpu.c:190-220,
@@ -325,6 +329,7 @@ int awefd__spher_set_model(awefd_model *m, const float *vel)
                 t[5][(long)ith * n1 + ir] = awefd_oneway_spher(vp[(long)(n2 - NOP - 1) * Y + ith * Z + ir], dt, dph);
             }
     }
+    if (!rc) rc = polar_oneway(m, t);
     for (int i = 0; i < 6; i++) {
         if (!rc) rc = up(&s->d_ow[i], t[i], sizeof(float) * sz[i]);
         free(t[i]);
@@ -359,6 +364,7 @@ int awefd__spher_set_receivers(awefd_model *m)
     }
     int rc = up(&s->d_rrtp, h, sizeof(int) * 3 * (m->nr > 0 ? m->nr : 1));
     free(h);
+    if (!rc) rc = polar_receivers(m);
     return rc ? rc : s->inj_dirty || !m->h_sj ? AWEFD_OK : build_conflicts(m);
 }
 
@@ -491,6 +497,7 @@ static int build_injection(awefd_model *m)
         rc = up(&s->d_inode, node, sizeof(long) * (nn > 0 ? nn : 1));
         if (!rc) rc = up(&s->d_ibeg, ibeg, sizeof(int) * (nn + 1));
         if (!rc) rc = up(&s->d_iw, iw, sizeof(float) * 2 * (n > 0 ? n : 1));
+        if (!rc) rc = polar_sources(m, node, nn);
     }
     free(e); free(node); free(ibeg); free(iw);
     if (!rc) s->inj_dirty = 0;
@@ -560,6 +567,249 @@ static void spher_args(const awefd_model *m, awefd_spher_args *a)
     memcpy(a->box, s->box, sizeof a->box);
     a->nconf = s->nconf;
     a->conf = s->d_conf;
+}
+
+/* ---- Resident polar loop (res_polar.hip) ---- */
+
+/* Last one-way rule at a node, as oneway_rule<2> (spher_kernels.hip):
+ * 0 none, 1 theta-low, 2 theta-high, 3 r-low, 4 r-high (spher_utils.c:518-563). */
+static int polar_rule(int ir, int ith, int n1, int n2)
+{
+    const int N = AWEFD_SPHER_NOP;
+    const int iop = ir < N ? ir : ir > n1 - N ? n1 - ir : ith < N ? ith : ith > n2 - N ? n2 - ith : 0;
+    int r = 0;
+    if (ith == N - iop) r = 1;
+    if (ith == n2 - N + iop - 1) r = 2;
+    if (ir == N - iop) r = 3;
+    if (ir == n1 - N + iop - 1) r = 4;
+    return r;
+}
+
+/* The one-way nodes every block of tile t computes, in one table: first the
+ * starts per block, then (16-byte aligned, at *off) the items.  ow: the
+ * coefficient tables of the four rules, or NULL (the count alone).  NULL:
+ * out of memory, or (*fits = 0) a block's list is too long or a chain too
+ * deep for the kernel. */
+static char *polar_items(const awefd_model *m, const awefd_res_tile *t, float *const ow[4], size_t *off,
+                         size_t *bytes, int *fits)
+{
+    static const int dr[5] = {0, 0, 0, 1, -1}, dt[5] = {0, 1, -1, 0, 0};
+    const int n1 = m->np[0], n2 = m->np[1], nb = m->nb, nblk = t->ntz * t->ntx, S = t->S;
+    char *h = NULL;
+    int *cnt = calloc((size_t)nblk + 1, sizeof(int));
+    *fits = 1;
+    *off = (sizeof(int) * (size_t)(nblk + 1) + 15) / 16 * 16;
+    for (int pass = 0; pass < 2 && cnt && *fits; pass++) {
+        for (int b = 0; pass == 0 && b < nblk; b++) cnt[b + 1] = 0;
+        for (int ith = 0; ith < n2; ith++)
+            for (int ir = 0; ir < n1; ir++) {
+                if (ir == 8 && ith >= 8 && ith < n2 - 8 && n1 > 16) ir = n1 - 8;    /* no rules inside */
+                const int k = polar_rule(ir, ith, n1, n2);
+                if (!k) continue;
+                const int r2 = ir + dr[k], t2 = ith + dt[k], k2 = polar_rule(r2, t2, n1, n2);
+                const int two = (k == 2 || k == 4) && k2;
+                const int r3 = r2 + dr[k2], t3 = t2 + dt[k2];
+                if (two && (k2 == 2 || k2 == 4) && polar_rule(r3, t3, n1, n2)) *fits = 0;
+                /* blocks whose computed nodes hold it: S - 1 beyond the owned */
+                const int e = S - 1;
+                for (int bx = (ith - e > 0 ? ith - e : 0) / t->ox; bx <= (ith + e) / t->ox && bx < t->ntx; bx++)
+                    for (int bz = (ir - e > 0 ? ir - e : 0) / t->zw; bz <= (ir + e) / t->zw && bz < t->ntz; bz++) {
+                        const int b = bz + t->ntz * bx;
+                        if (pass == 0) {
+                            cnt[b + 1]++;
+                            continue;
+                        }
+                        const int zo = bz * t->zw - S, xo = bx * t->ox - S;
+#define AT(r, th) (((th) - xo) * 64 + (r) - zo)
+                        awefd_polar_item *q = (awefd_polar_item *)(h + *off) + cnt[b]++;
+                        q->off = AT(ir, ith);
+                        q->noff = AT(r2, t2);
+                        q->nnoff = two ? AT(r3, t3) : -1;
+#undef AT
+                        q->b = ow[k - 1][k <= 2 ? ir : ith];
+                        q->b2 = two ? ow[k2 - 1][k2 <= 2 ? r2 : t2] : 0.f;
+                        q->zero = m->p.fsrf && ir > n1 - nb;
+                        const int di = ir < nb ? nb - ir : ith < nb ? nb - ith : ir > n1 - nb ? ir - (n1 - nb)
+                                       : ith > n2 - nb ? ith - (n2 - nb) : -1;
+                        q->damp = di >= 0 ? awefd_spher_damp(di, nb) : 1.0;
+                    }
+            }
+        if (pass == 0) {
+            for (int b = 0; b < nblk; b++) {
+                if (cnt[b + 1] > AWEFD_POLAR_ITEMS) *fits = 0;
+                cnt[b + 1] += cnt[b];
+            }
+            *bytes = *off + sizeof(awefd_polar_item) * (size_t)(cnt[nblk] > 0 ? cnt[nblk] : 1);
+            if (!ow || !*fits) break;
+            if (!(h = malloc(*bytes))) break;
+            memcpy(h, cnt, sizeof(int) * (size_t)(nblk + 1));
+        }
+    }
+    free(cnt);
+    return h;
+}
+
+/* Whether this grid takes the resident loop, and its tile: the fewest rows
+ * per wave whose blocks fit one per CU, two steps per exchange where a tile
+ * of them does.  The tiles at the high faces must hold a one-way node's
+ * chain.  AWEFD_RESIDENT=0, AWEFD_RES_STEPS=1 or 2: as for the cartesian
+ * loop. */
+static int polar_create(awefd_model *m)
+{
+    static const int rx2[] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 0}, rx1[] = {2, 3, 4, 6, 8, 0};
+    awefd_res *r = &m->res;
+    const char *on = getenv("AWEFD_RESIDENT"), *st = getenv("AWEFD_RES_STEPS");
+    int cus = 0, coop = 0;
+    if (m->ndim != 2 || (on && atoi(on) == 0)) return AWEFD_OK;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev) != hipSuccess ||
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, m->dev) != hipSuccess || !coop)
+        return AWEFD_OK;
+    for (int S = 2; S >= 1; S--) {
+        if (st && atoi(st) != S) continue;
+        for (const int *rx = S == 2 ? rx2 : rx1; *rx; rx++) {
+            awefd__res_tile_of(m, 1, *rx, S, &r->t);
+            const awefd_res_tile *t = &r->t;
+            const int lz = m->np[0] - (t->ntz - 1) * t->zw, lx = m->np[1] - (t->ntx - 1) * t->ox;
+            size_t off, bytes;
+            int fits;
+            if (!t->on || (long)t->ntz * t->ntx > cus || (t->ntz > 1 && lz < AWEFD_POLAR_FACE) ||
+                (t->ntx > 1 && (lx < AWEFD_POLAR_FACE || t->ox < AWEFD_POLAR_FACE)))
+                continue;
+            free(polar_items(m, t, NULL, &off, &bytes, &fits));
+            if (!fits || awefd__polar_blocks(*rx, S) < 1) continue;
+            return awefd__res_buffers(m);
+        }
+    }
+    return AWEFD_OK;
+}
+
+static int polar_oneway(awefd_model *m, float *const t[4])
+{
+    awefd_res *r = &m->res;
+    size_t bytes;
+    int fits;
+    if (!r->on) return AWEFD_OK;
+    char *h = polar_items(m, &r->t, t, &r->one_off, &bytes, &fits);
+    if (!h) return awefd__fail(AWEFD_ENOMEM, "one-way nodes");
+    int rc = awefd__res_grow(&r->one, bytes);
+    hipError_t e = rc ? hipSuccess : hipMemcpy(r->one.p, h, bytes, hipMemcpyHostToDevice);
+    free(h);
+    return rc || e == hipSuccess ? rc : awefd__fail(AWEFD_EHIP, "one-way nodes: %s", hipGetErrorString(e));
+}
+
+/* Injection nodes of every block's image (image offset, node number). */
+static int polar_sources(awefd_model *m, const long *node, int n)
+{
+    awefd_res *r = &m->res;
+    const awefd_res_tile *t = &r->t;
+    if (!r->on) return AWEFD_OK;
+    const int nblk = t->ntz * t->ntx, S = t->S;
+    const size_t head = sizeof(int) * (size_t)(nblk + 1);
+    int *beg = calloc((size_t)nblk + 1, sizeof(int)), *h = NULL;
+    int rc = beg ? AWEFD_OK : awefd__fail(AWEFD_ENOMEM, "resident source table");
+    for (int pass = 0; pass < 2 && !rc; pass++) {
+        for (int i = 0; i < n; i++) {
+            const int ir = (int)(node[i] % m->ld), ith = (int)(node[i] / m->ld);
+            for (int bx = (ith - S > 0 ? ith - S : 0) / t->ox; bx <= (ith + S) / t->ox && bx < t->ntx; bx++)
+                for (int bz = (ir - S > 0 ? ir - S : 0) / t->zw; bz <= (ir + S) / t->zw && bz < t->ntz; bz++) {
+                    const int b = bz + t->ntz * bx, z = ir - (bz * t->zw - S), x = ith - (bx * t->ox - S);
+                    if (z < 0 || z >= t->zw + 2 * S || x < 0 || x >= t->ox + 2 * S) continue;
+                    if (pass == 0) {
+                        beg[b + 1]++;
+                    } else {
+                        int *q = h + nblk + 1 + 2 * (size_t)beg[b]++;
+                        q[0] = x * 64 + z;
+                        q[1] = i;
+                    }
+                }
+        }
+        if (pass == 0) {
+            for (int b = 0; b < nblk; b++) beg[b + 1] += beg[b];
+            if (!(h = malloc(head + sizeof(int) * 2 * (size_t)(beg[nblk] > 0 ? beg[nblk] : 1))))
+                rc = awefd__fail(AWEFD_ENOMEM, "resident source table");
+            else memcpy(h, beg, head);
+        }
+    }
+    if (!rc) {
+        const size_t bytes = head + sizeof(int) * 2 * (size_t)(h[nblk] > 0 ? h[nblk] : 1);
+        rc = awefd__res_grow(&r->src, bytes);
+        hipError_t e = rc ? hipSuccess : hipMemcpy(r->src.p, h, bytes, hipMemcpyHostToDevice);
+        if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident source table: %s", hipGetErrorString(e));
+        r->inj_off = head;
+    }
+    free(beg);
+    free(h);
+    return rc;
+}
+
+/* Receivers per block, by the block that owns their first corner. */
+static int polar_receivers(awefd_model *m)
+{
+    awefd_res *r = &m->res;
+    const awefd_res_tile *t = &r->t;
+    if (!r->on) return AWEFD_OK;
+    const int nr = m->nr, nblk = t->ntz * t->ntx;
+    const size_t bytes = sizeof(int) * ((size_t)nblk + 1 + (nr > 0 ? nr : 1));
+    int *h = calloc(1, bytes), *fill = malloc(sizeof(int) * (size_t)nblk);
+    int rc = h && fill ? AWEFD_OK : awefd__fail(AWEFD_ENOMEM, "resident receiver table");
+#define BLOCK(i) (m->h_rj[3 * (i) + 1] / t->zw + t->ntz * (m->h_rj[3 * (i)] / t->ox))
+    for (int i = 0; i < nr && !rc; i++) h[BLOCK(i) + 1]++;
+    for (int b = 0; b < nblk && !rc; b++) h[b + 1] += h[b];
+    if (!rc) memcpy(fill, h, sizeof(int) * (size_t)nblk);
+    for (int i = 0; i < nr && !rc; i++) h[nblk + 1 + fill[BLOCK(i)]++] = i;
+#undef BLOCK
+    if (!rc) rc = awefd__res_grow(&r->rec, bytes);
+    hipError_t e = rc ? hipSuccess : hipMemcpy(r->rec.p, h, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident receiver table: %s", hipGetErrorString(e));
+    r->idx_off = sizeof(int) * ((size_t)nblk + 1);
+    free(h);
+    free(fill);
+    return rc;
+}
+
+/* The whole loop of a set-up model; *done = 0: not taken, the caller runs the
+ * other loop from the start. */
+int awefd__polar_run(awefd_model *m, float *dtr, int *done)
+{
+    spher_state *s = st(m);
+    awefd_res *r = &m->res;
+    awefd_polar_args a;
+    int rc;
+    *done = 0;
+    if (s->inj_dirty && (rc = build_injection(m))) return rc;
+    if (!s->d_rrtp) return awefd__fail(AWEFD_ESTATE, "receivers not set");
+    memset(&a, 0, sizeof a);
+    a.n1 = m->np[0];
+    a.n2 = m->np[1];
+    a.ld = m->ld;
+    a.ntz = r->t.ntz;
+    a.ntx = r->t.ntx;
+    a.nb = m->nb;
+    a.fsrf = m->p.fsrf;
+    a.pc = s->d_pc;
+    a.vv = m->dvel;
+    a.damp = m->d_damp;
+    a.P = m->dP;
+    a.C = m->dC;
+    a.nt = m->p.nt;
+    a.sbeg = (const int *)r->src.p;
+    a.snode = (const int *)((const char *)r->src.p + r->inj_off);
+    a.ibeg = s->d_ibeg;
+    a.iw = s->d_iw;
+    a.wav = m->d_wav;
+    a.obeg = (const int *)r->one.p;
+    a.items = (const awefd_polar_item *)((const char *)r->one.p + r->one_off);
+    a.nr = m->nr;
+    a.rbeg = (const int *)r->rec.p;
+    a.ridx = (const int *)((const char *)r->rec.p + r->idx_off);
+    a.rj = s->d_rrtp;
+    a.rw = m->d_rw;
+    a.tr = dtr;
+    a.E = (unsigned long long *)r->E.p;
+    a.stop = r->stop;
+    awefd__res_wait(&a.wmask, &a.wticks);
+    if ((rc = awefd__res_tags(&r->E, &r->tag, a.nt, m->stream, &a.tag0))) return rc;
+    return awefd__res_finish(m, awefd__polar_launch(&a, r->t.ntz * r->t.ntx, r->t.rx, r->t.S, m->stream), done);
 }
 
 /* The time loop (MAWEFDspher2Dcpu.c:264-317, MAWEFDspher3Dcpu.c:302-359).
