@@ -208,7 +208,7 @@ int awefd_batch_set_depth(awefd_batch *b, int depth);
 int awefd_batch_tune_depth(awefd_batch *b, int steps, int *rx_out, int *group_mb_out, int *depth_out,
                            double *ms_out);
 /* The batch's awefd_run_ckpt: every shot's forward loop with checkpoints
- * every ckpt steps (<= 0: ceil(sqrt(nt))), one graph.  Traces as after
+ * every ckpt steps (<= 0: as awefd_run_ckpt, for the shots together), one graph.  Traces as after
  * awefd_batch_run. */
 int awefd_batch_run_ckpt(awefd_batch *b, int ckpt);
 /* Sum over the shots of awefd_adjoint_grad, every shot's backward pass in
@@ -224,8 +224,11 @@ int awefd_batch_adjoint_grad(awefd_batch *b, const float *const *d_res, float *d
  * traces d of a cartesian 2-D loop, s = 1/v^2 on the model grid. ---- */
 
 /* The forward loop of awefd_run_dev (same traces, same final fields) that
- * also keeps the field pair of every ckpt-th step (<= 0: ceil(sqrt(nt))) in
- * device memory for awefd_adjoint_grad: 2 ceil(nt/ckpt) padded fields.
+ * also keeps the field pair of every ckpt-th step in device memory for
+ * awefd_adjoint_grad: 2 ceil(nt/ckpt) padded fields.  With ckpt >= nt it keeps
+ * every field (nt + 1 padded ones) and nothing is recomputed; ckpt <= 0 does
+ * so while three quarters of the card's memory stay free, else takes
+ * ceil(sqrt(nt)).  The gradient's bits do not depend on ckpt.
  * AWEFD_CART2D with constant density only. */
 int awefd_run_ckpt(awefd_model *m, float *d_traces, int ckpt);
 /* dJ/ds at the model of the last awefd_run_ckpt (AWEFD_ESTATE if a setter

@@ -253,7 +253,8 @@ class Batch:
 
     def run_ckpt(self, ckpt=0):
         """Every shot's forward loop keeping checkpoints every ``ckpt`` steps
-        (0: ceil(sqrt(nt))) for adjoint_grad."""
+        (0: every field while memory is ample, else ceil(sqrt(nt))) for
+        adjoint_grad."""
         L.check(self.lib.awefd_batch_run_ckpt(self.h, int(ckpt)))
 
     def adjoint_grad(self, res_ptrs, grad_ptr):

@@ -11,7 +11,9 @@
  * buffers (out-of-place steps, so the checkpoint survives and no copies are
  * made) and steps the adjoint backwards through them (four adjoint fields
  * in rotation and the dJ/dV accumulator).  Fields held: 2 ceil(nt/K)
- * checkpoints + K-1 segment buffers + 5.
+ * checkpoints + K-1 segment buffers + 5.  With K = nt the one segment is the
+ * whole run: the forward run stores its fields there and nothing is
+ * recomputed.
  */
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
@@ -170,12 +172,31 @@ static adj_state *state(const awefd_model *m)
     return (adj_state *)m->adj;
 }
 
+/* Checkpoint interval when the caller names none (ckpt <= 0): nt, every field
+ * kept by the forward run and none recomputed, while at least three quarters
+ * of the card's memory stays free beside the n models' fields; else
+ * ceil(sqrt(nt)).  Keeping them takes a quarter of a gradient's steps away. */
+int awefd__adj_interval(awefd_model *const *ms, int n, int ckpt)
+{
+    const int nt = ms[0]->p.nt;
+    size_t need = 0, fr = 0, total = 0;
+    if (ckpt > 0) return ckpt < nt ? ckpt : nt;
+    for (int i = 0; i < n; i++) {
+        const adj_state *s = state(ms[i]);
+        if (!(s && s->K == nt && s->seg)) need += sizeof(float) * (size_t)ms[i]->nalloc * (size_t)(nt + 1);
+    }
+    if (need == 0) return nt;
+    if (hipSetDevice(ms[0]->dev) == hipSuccess && hipMemGetInfo(&fr, &total) == hipSuccess && fr >= need + total / 4 * 3)
+        return nt;
+    return (int)ceil(sqrt((double)nt));
+}
+
 int awefd__adj_ckpt_setup(awefd_model *m, int ckpt)
 {
     int rc = check_model(m, "checkpointed run");
     if (rc) return rc;
     const int nt = m->p.nt;
-    const int K = ckpt > 0 ? (ckpt < nt ? ckpt : nt) : (int)ceil(sqrt((double)nt));
+    const int K = awefd__adj_interval(&m, 1, ckpt);
     const int nck = (nt + K - 1) / K;
     if ((size_t)m->nalloc * 4 >= 0x80000000u)
         return awefd__fail(AWEFD_EINVAL, "gradient: field of %ld nodes exceeds 2 GiB", m->nalloc);
@@ -194,7 +215,73 @@ int awefd__adj_ckpt_setup(awefd_model *m, int ckpt)
         s->K = K;
         s->nck = nck;
     }
-    return dev_alloc(&s->ck, sizeof(float) * (size_t)m->nalloc * 2 * nck);
+    if ((rc = dev_alloc(&s->ck, sizeof(float) * (size_t)m->nalloc * 2 * nck))) return rc;
+    /* one segment: the forward run stores its fields */
+    if (K < nt || K == 1 || !(rc = dev_alloc(&s->seg, sizeof(float) * (size_t)m->nalloc * (K - 1)))) return AWEFD_OK;
+    const int few = (int)ceil(sqrt((double)nt));
+    return ckpt > 0 || few == nt ? rc : awefd__adj_ckpt_setup(m, few);
+}
+
+/* Field n of a run that keeps them all; n = -1: the one before the first. */
+static float *kept_field(const adj_state *s, long nalloc, int n)
+{
+    return n < 0 ? s->ck + nalloc : n == 0 ? s->ck : s->seg + (size_t)(n - 1) * nalloc;
+}
+
+/* The last step of a run that kept fields 0 .. nt-1, and the model's field
+ * pair as its loop leaves it. */
+int awefd__adj_kept_end(awefd_model *m, hipStream_t stream)
+{
+    const adj_state *s = state(m);
+    const int nt = m->p.nt;
+    awefd_cart_args a;
+    awefd__cart_args(m, &a);
+    a.nr = 0;
+    a.C = kept_field(s, m->nalloc, nt - 1);
+    a.P = kept_field(s, m->nalloc, nt - 2);
+    a.Pn = m->dC;
+    a.it = nt - 1;
+    const int e = awefd_launch_cart_step(&a, m->nop, 2, m->p.sse, 0, stream);
+    if (e) return awefd__fail(AWEFD_EHIP, "step %d launch: %s", nt - 1, hipGetErrorString((hipError_t)e));
+    const hipError_t he = hipMemcpyAsync(m->dP, a.C, sizeof(float) * (size_t)m->nalloc, hipMemcpyDeviceToDevice, stream);
+    if (he != hipSuccess) return awefd__fail(AWEFD_EHIP, "last field: %s", hipGetErrorString(he));
+    m->steps_done = nt;
+    return AWEFD_OK;
+}
+
+/* Traces of a run that kept fields 0 .. nt-1. */
+int awefd__adj_kept_traces(awefd_model *m, float *dtr, hipStream_t stream)
+{
+    const adj_state *s = state(m);
+    awefd_cart_args a;
+    awefd__cart_args(m, &a);
+    const int e = awefd_launch_cart_traces(&a, s->ck, s->seg, m->nalloc, m->p.nt, dtr, stream);
+    return e ? awefd__fail(AWEFD_EHIP, "traces: %s", hipGetErrorString((hipError_t)e)) : AWEFD_OK;
+}
+
+/* Forward run that keeps every field: the resident loop where the model takes
+ * it, else out-of-place steps and one launch for the traces. */
+static int run_kept(awefd_model *m, float *dtr)
+{
+    adj_state *s = state(m);
+    const int nt = m->p.nt;
+    int rc = AWEFD_OK, e = awefd_launch_fill(s->ck, 2 * m->nalloc, 0.f, m->stream), done = 0;
+    if (e) return awefd__fail(AWEFD_EHIP, "gradient reset: %s", hipGetErrorString((hipError_t)e));
+    if (m->res.on && !m->prof && ((rc = awefd__res_run(m, dtr, s->seg, &done)) || done)) return rc;
+    awefd_cart_args a;
+    awefd__cart_args(m, &a);
+    a.nr = 0;
+    for (int n = 0; n + 1 < nt; n++) {
+        a.C = kept_field(s, m->nalloc, n);
+        a.P = kept_field(s, m->nalloc, n - 1);
+        a.Pn = kept_field(s, m->nalloc, n + 1);
+        a.it = n;
+        if ((e = awefd_launch_cart_step(&a, m->nop, 2, m->p.sse, 0, m->stream)))
+            return awefd__fail(AWEFD_EHIP, "step %d launch: %s", n, hipGetErrorString((hipError_t)e));
+    }
+    if ((rc = awefd__adj_kept_end(m, m->stream)) || (rc = awefd__adj_kept_traces(m, dtr, m->stream))) return rc;
+    const hipError_t he = hipStreamSynchronize(m->stream);
+    return he == hipSuccess ? AWEFD_OK : awefd__fail(AWEFD_EHIP, "forward run: %s", hipGetErrorString(he));
 }
 
 float *awefd__adj_ckpt(const awefd_model *m, int k)
@@ -234,6 +321,10 @@ int awefd_run_ckpt(awefd_model *m, float *d_traces, int ckpt)
     const size_t fb = sizeof(float) * (size_t)m->nalloc;
     awefd_cart_args a;
     if ((rc = awefd__ensure_traces(m))) goto done;
+    if (K == nt) {
+        if (!(rc = run_kept(m, d_traces ? d_traces : m->d_traces))) awefd__adj_mark(m);
+        goto done;
+    }
     if ((rc = awefd_reset(m))) goto done;
     awefd__cart_args(m, &a);
     for (int it = 0; it < nt; it++) {
@@ -431,7 +522,7 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
         const int n0 = k * K, n1 = n0 + K < nt ? n0 + K : nt;
         float *ckc = awefd__adj_ckpt(m, k), *ckp = ckc + m->nalloc;
 #define FIELD(n) ((n) == n0 ? ckc : s->seg + (size_t)((n) - n0 - 1) * m->nalloc)
-        for (int n = n0; n + 1 < n1; n++) {
+        for (int n = n0; n + 1 < n1 && K < nt; n++) {
             a.C = FIELD(n);
             a.P = n == n0 ? ckp : FIELD(n - 1);
             a.Pn = FIELD(n + 1);
@@ -443,6 +534,8 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
             }
         }
 #undef FIELD
+        /* (in pairs, as the batch takes them, a 400 x 800 shot's 203 blocks
+         * need 22 us a pair against 2 x 7.4) */
         for (int n = n1 - 1; n >= n0; n--) {
             int e = awefd_launch_adj2d_step(&g, n, m->nop, m->stream);
             if (e) {

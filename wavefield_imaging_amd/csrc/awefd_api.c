@@ -1121,7 +1121,7 @@ static int run_common(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
     if (whole2d && m->res.on) {
         /* the resident loops start from zero fields of their own */
         int done;
-        rc = is_cart(m) ? awefd__res_run(m, trow0, &done) : awefd__polar_run(m, trow0, &done);
+        rc = is_cart(m) ? awefd__res_run(m, trow0, NULL, &done) : awefd__polar_run(m, trow0, &done);
         if (rc || done) return rc;
     }
     if ((rc = awefd_reset(m))) return rc;

@@ -19,6 +19,7 @@
  */
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
+#include <math.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -1135,13 +1136,72 @@ static int capture_fwd(awefd_batch *b, int depth)
     return AWEFD_OK;
 }
 
+/* The forward run of every shot with every field kept: the segment's
+ * recompute passes from the first step on, as one graph, then per shot the
+ * last step and the traces from the stored fields. */
+static int run_kept(awefd_batch *b)
+{
+    const int depth = ckpt_depth(b), nt = b->nt;
+    int rc = AWEFD_OK;
+    if (depth == 3 && (!b->t2_ok || b->t2_depth != 3) && (rc = t2_build(b, 3))) return rc;
+    for (int s = 0; s < b->nshot; s++) awefd__adj_cart_ckpt(b->m[s], &b->h[s]);
+    HIPCHK(hipMemcpy(b->d_shots, b->h, sizeof(*b->h) * b->nshot, hipMemcpyHostToDevice));
+    if (!(b->xfwd && b->fwd_ok && b->fwd_depth == depth)) {
+        if (b->xfwd) hipGraphExecDestroy(b->xfwd);
+        if (b->gfwd) hipGraphDestroy(b->gfwd);
+        b->xfwd = NULL;
+        b->gfwd = NULL;
+        HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+        int e = 0;
+        for (int s = 0; s < b->nshot && !e; s++)
+            e = awefd_launch_fill(awefd__adj_ckpt(b->m[s], 0), 2 * b->m[s]->nalloc, 0.f, b->stream);
+        for (int g = 0; g < b->ngroup && !e; g++) {
+            int n = 0;
+            for (; depth == 3 && n + 3 <= nt - 1 && !e; n += 3)
+                e = awefd_launch_cart_batch_t3rc(b->d_shots, b->d_bshot2 + b->goff2[g], b->gnblk2[g], n, b->nop, b->sse,
+                                                 b->rx, b->stream);
+            for (; n + 1 < nt && !e; n++)
+                e = awefd_launch_cart_batch_rc(b->d_shots, b->d_bshot + b->goff[g], b->gnblk[g], n, b->nop, b->sse,
+                                               b->rx, b->stream);
+        }
+        if (e) rc = awefd__fail(AWEFD_EHIP, "batched forward run: %s", hipGetErrorString((hipError_t)e));
+        hipGraph_t gr = NULL;
+        hipError_t he = hipStreamEndCapture(b->stream, &gr);
+        if (rc) {
+            if (gr) hipGraphDestroy(gr);
+            return rc;
+        }
+        if (he != hipSuccess) return awefd__fail(AWEFD_EHIP, "batched forward capture: %s", hipGetErrorString(he));
+        b->gfwd = gr;
+        HIPCHK(hipGraphInstantiate(&b->xfwd, gr, NULL, NULL, 0));
+        b->fwd_ok = 1;
+        b->fwd_depth = depth;
+    }
+    for (int s = 0; s < b->nshot; s++) b->fwd_ck[s] = awefd__adj_ckpt(b->m[s], 0);
+    HIPCHK(hipGraphLaunch(b->xfwd, b->stream));
+    for (int s = 0; s < b->nshot; s++) {
+        awefd_model *m = b->m[s];
+        if ((rc = awefd__adj_kept_end(m, b->stream)) || (rc = awefd__adj_kept_traces(m, m->d_traces, b->stream))) return rc;
+    }
+    HIPCHK(hipStreamSynchronize(b->stream));
+    for (int s = 0; s < b->nshot; s++) awefd__adj_mark(b->m[s]);
+    return AWEFD_OK;
+}
+
 int awefd_batch_run_ckpt(awefd_batch *b, int ckpt)
 {
     if (!b) return awefd__fail(AWEFD_EINVAL, "NULL batch");
     HIPCHK(hipSetDevice(b->dev));
     int rc;
+    if ((rc = shots_ready(b))) return rc;
+    int want = awefd__adj_interval(b->m, b->nshot, ckpt);
     for (int s = 0; s < b->nshot; s++)
-        if ((rc = awefd__adj_ckpt_setup(b->m[s], ckpt))) return rc;
+        if ((rc = awefd__adj_ckpt_setup(b->m[s], want))) {
+            const int few = (int)ceil(sqrt((double)b->nt));
+            if (ckpt > 0 || want == few) return rc;
+            want = few;                      /* no memory for every field */
+            s = -1;
+        }
     const int K = awefd__adj_K(b->m[0]);
     if ((rc = batch_sync(b))) return rc;
     if (K != b->K) {
@@ -1154,6 +1214,7 @@ int awefd_batch_run_ckpt(awefd_batch *b, int ckpt)
         return awefd__fail(AWEFD_ENOMEM, "batch checkpoint bases");
     for (int s = 0; s < b->nshot; s++)
         if (b->fwd_ck[s] != awefd__adj_ckpt(b->m[s], 0)) b->fwd_ok = 0;
+    if (K == b->nt) return run_kept(b);
     const int depth = ckpt_depth(b);
     if ((rc = capture_fwd(b, depth))) return rc;
     for (int s = 0; s < b->nshot; s++) b->fwd_ck[s] = awefd__adj_ckpt(b->m[s], 0);
@@ -1298,7 +1359,8 @@ static int capture_bwd(awefd_batch *b, int depth, int adepth)
     for (int g = 0; g < b->ngroup && !e; g++)
         for (int k = b->nck - 1; k >= 0 && !e; k--) {
             const int n0 = k * b->K, n1 = n0 + b->K < b->nt ? n0 + b->K : b->nt;
-            int n = n0;
+            /* K = nt: the forward run kept the segment's fields */
+            int n = b->K < b->nt ? n0 : n1;
             for (; depth == 3 && n + 3 <= n1 - 1 && !e; n += 3)
                 e = awefd_launch_cart_batch_t3rc(b->d_shots, b->d_bshot2 + b->goff2[g], b->gnblk2[g], n, b->nop,
                                                  b->sse, b->rx, b->stream);

@@ -175,6 +175,9 @@ typedef struct {
     const int *rj;
     const float *rw;
     float *tr;                   /* traces, nt x nr                            */
+    /* not NULL: field it + 1 goes to F + it nal for it + 1 < nt               */
+    float *F;
+    long nal;
     /* rim words (two parities of ntz ntx rims), tag of step 0, and the flag a
      * block raises when it gives up waiting */
     unsigned long long *E;
@@ -408,6 +411,10 @@ int awefd__polar_blocks(int rx, int S);
 /* Launchers (cart_kernels.hip).  Return 0 or a HIP error code. */
 int awefd_launch_cart_step(const awefd_cart_args *a, int nop, int ndim, int sse, int varden,
                            void *stream);
+/* trace rows 0..nt-1 of a 2-D grid whose current fields are all stored: row 0
+ * from c0, row n from seg + (n - 1) nal; traces nt x a->nr */
+int awefd_launch_cart_traces(const awefd_cart_args *a, const float *c0, const float *seg, long nal, int nt,
+                             float *traces, void *stream);
 int awefd_launch_cart_abc_xy(const awefd_cart_args *a, int nop, void *stream);
 /* hybrid boundary of the new field P (apply_abc): z lines, x lines, then in
  * 3-D y lines, each face of a line swept by one thread */

@@ -148,7 +148,7 @@ int  awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf
 int  awefd__res_tags(awefd_res_buf *E, unsigned *tag, int nt, hipStream_t s, unsigned *tag0);
 void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_res_buf *src, size_t inj_off,
                      const awefd_res_buf *rec, size_t idx_off, float *dtr, awefd_res_args *a);
-int  awefd__res_run(awefd_model *m, float *dtr, int *done);
+int  awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done);
 int  awefd__res_grow(awefd_res_buf *b, size_t bytes);
 void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_tile *t);
 int  awefd__res_buffers(awefd_model *m);
@@ -160,6 +160,9 @@ int  awefd__polar_run(awefd_model *m, float *dtr, int *done);
 /* gradient internals shared with the batched path (awefd_adjoint.c) */
 void   awefd__adjoint_free(awefd_model *m);
 int    awefd__adj_ckpt_setup(awefd_model *m, int ckpt);
+int    awefd__adj_interval(awefd_model *const *ms, int n, int ckpt);
+int    awefd__adj_kept_end(awefd_model *m, hipStream_t stream);
+int    awefd__adj_kept_traces(awefd_model *m, float *dtr, hipStream_t stream);
 float *awefd__adj_ckpt(const awefd_model *m, int k);
 int    awefd__adj_K(const awefd_model *m);
 void   awefd__adj_mark(awefd_model *m);

@@ -318,15 +318,18 @@ int awefd__res_finish(awefd_model *m, int launched, int *done)
     return AWEFD_OK;
 }
 
-/* The whole loop of a set-up model; *done = 0: not taken (or given up on
- * waiting for a block), the caller runs the other loop from the start. */
-int awefd__res_run(awefd_model *m, float *dtr, int *done)
+/* The whole loop of a set-up model, with its fields 1 .. nt-1 into `fields`
+ * (not NULL); *done = 0: not taken (or given up on waiting for a block), the
+ * caller runs the other loop from the start. */
+int awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done)
 {
     awefd_res *r = &m->res;
     awefd_res_args a;
     *done = 0;
     if (!r->on) return AWEFD_OK;
     awefd__res_args(m, &r->t, &r->src, r->inj_off, &r->rec, r->idx_off, dtr, &a);
+    a.F = fields;
+    a.nal = m->nalloc;
     const int vd = a.rho != NULL;
     if (vd && awefd__res_blocks(m->nop, &r->t, 1) < 1) return AWEFD_OK;   /* too many rows for the records */
     a.E = (unsigned long long *)r->E.p;

@@ -879,6 +879,15 @@ __global__ __launch_bounds__(step_nw<NARROW>() * WAVE) void k_cart_step(const aw
                                                                             dst);
 }
 
+/* The trace rows of a 2-D grid whose current fields are all stored, one row
+ * per grid row of blocks (256 rows of 2,000 receivers: 24 us). */
+__global__ __launch_bounds__(256) void k_cart_traces(const awefd_cart_args a, const float *c0, const float *seg, long nal,
+                                                     float *traces)
+{
+    const int n = blockIdx.y;
+    cart_extract<2>(a, n == 0 ? c0 : seg + (n - 1) * nal, traces + (long)n * a.nr, blockIdx.x * 256 + threadIdx.x);
+}
+
 /* The batched 2-D step kernel: one launch advances every shot of a batch one
  * time step.  Each shot's arguments live in device memory; block b belongs
  * to shot bshot[b] and is that shot's block b - blk0 (stencil tiles, then
@@ -1815,6 +1824,15 @@ extern "C" int awefd_launch_cart_hybrid(const awefd_cart_args *a, int nop, int n
     hipLaunchKernelGGL(k_cart_hybrid<1>, dim3((unsigned)((2 * nl[1] + 255) / 256)), dim3(256), 0, s, *a, nop);
     if (ndim == 3)
         hipLaunchKernelGGL(k_cart_hybrid<2>, dim3((unsigned)((2 * nl[2] + 255) / 256)), dim3(256), 0, s, *a, nop);
+    return (int)hipGetLastError();
+}
+
+extern "C" int awefd_launch_cart_traces(const awefd_cart_args *a, const float *c0, const float *seg, long nal, int nt,
+                                        float *traces, void *stream)
+{
+    if (a->nr <= 0 || nt <= 0) return 0;
+    hipLaunchKernelGGL(k_cart_traces, dim3((a->nr + 255) / 256, nt), dim3(256), 0, (hipStream_t)stream, *a, c0, seg, nal,
+                       traces);
     return (int)hipGetLastError();
 }
 

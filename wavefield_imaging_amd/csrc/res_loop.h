@@ -344,6 +344,18 @@ __global__ __launch_bounds__(NTHR) void k_cart2d_res(const awefd_res_args, const
                 }
             amp = na;
         }
+        /* the gradient keeps every field: the owned nodes, stored and not
+         * waited for */
+        if (__builtin_expect(a.F != nullptr, 0) && it + 1 < nt) {
+            const rsrc_t rF = mk_rsrc(a.F + (long)it * a.nal, (unsigned)n2 * rowb);
+#pragma unroll
+            for (int j = 0; j < RX; j++) {
+                const int lr = wv * RX + j;
+                const bool in = lr >= EXT && lr < EXT + OX && x0 + j < n2;
+                bst<2>(rF, in && own ? (unsigned)iz * 4u : OOB, in ? (unsigned)(x0 + j) * rowb : 0u,
+                       ne > 0 ? N[j * WAVE + lane] : p[NOP + j]);
+            }
+        }
         /* between exchanges the image of this step is overwritten next */
         if (S > 1 && XCH && nrec > 0) extract(I, it);
         if (XCH) dead = __builtin_amdgcn_readfirstlane(dead);
