@@ -22,6 +22,7 @@
 #include <string.h>
 
 #include "awefd_model.h"
+#include "res_adj.h"
 #include "awefd_setup.h"
 
 #define HIPCHK(call)                                                                        \
@@ -50,6 +51,13 @@ typedef struct {
     int lists_ok;
     awefd_adj2d_args *d_args; /* device copy of the kernel arguments    */
     float *ones;              /* sponge table of ones (runs without dabc) */
+    /* resident adjoint loop (res_adj.hip): its tile, rim words and, per wave,
+     * its receiver and injection nodes */
+    awefd_res_tile rt;
+    awefd_res_buf E;
+    unsigned tag;
+    awefd_inj *rinjr, *sinjr;
+    int *rbegr, *sbegr;
 } adj_state;
 
 static void free_lists(adj_state *s)
@@ -57,6 +65,9 @@ static void free_lists(adj_state *s)
     hipFree(s->rinj); hipFree(s->sinj); hipFree(s->rbeg); hipFree(s->sbeg);
     hipFree(s->rinjb); hipFree(s->sinjb); hipFree(s->rbegb); hipFree(s->sbegb);
     hipFree(s->rinj2); hipFree(s->sinj2); hipFree(s->rbeg2); hipFree(s->sbeg2);
+    hipFree(s->rinjr); hipFree(s->sinjr); hipFree(s->rbegr); hipFree(s->sbegr);
+    s->rinjr = s->sinjr = NULL;
+    s->rbegr = s->sbegr = NULL;
     s->rinj = s->sinj = s->rinjb = s->sinjb = s->rinj2 = s->sinj2 = NULL;
     s->rbeg = s->sbeg = s->rbegb = s->sbegb = s->rbeg2 = s->sbeg2 = NULL;
     s->lists_ok = 0;
@@ -70,6 +81,7 @@ void awefd__adjoint_free(awefd_model *m)
     hipFree(s->ck); hipFree(s->seg);
     hipFree(s->A[0]); hipFree(s->A[1]); hipFree(s->A[2]); hipFree(s->A[3]); hipFree(s->gV); hipFree(s->d_args);
     hipFree(s->ones);
+    hipFree(s->E.p);
     free_lists(s);
     free(s);
     m->adj = NULL;
@@ -87,13 +99,13 @@ static int min_i(int a, int b)
 
 /* Interpolation points of a 2-D grid as (node, id, weight) entries bucketed
  * per tile, uploaded to the device.  id is the point index (receivers) or
- * the wavelet column (sources: 0 with expl).  ov = 0: tiles of 64 x tx
+ * the wavelet column (sources: 0 with expl).  ov = 0: tiles of tz x tx
  * nodes, each node in one; ov = nop: the two-step pass's tiles, whose
  * outputs are (64 - 2 ov) x (tx - 2 ov) nodes and whose extent reaches ov
  * beyond them, each node in every tile whose extent holds it (at most two
  * per axis). */
 static int point_buckets(const awefd_model *m, int n, const int *j, const float *w, int same_id, int ntz,
-                         int ntx, int tx, int ov, awefd_inj **d_inj, int **d_beg)
+                         int ntx, int tz, int tx, int ov, awefd_inj **d_inj, int **d_beg)
 {
     const long cap = (ov ? 16L : 4L) * n;
     const int nbucket = ntz * ntx, sz = 64 - 2 * ov, sx = tx - 2 * ov;
@@ -115,7 +127,7 @@ static int point_buckets(const awefd_model *m, int n, const int *j, const float 
                 en.w3 = 1.f;
                 if (!ov) {
                     keys[ne].e = en;
-                    keys[ne++].bucket = en.z / 64 + ntz * (en.x / tx);
+                    keys[ne++].bucket = en.z / tz + ntz * (en.x / tx);
                     continue;
                 }
                 /* tile t's extent: [t s - ov, t s - ov + width) */
@@ -362,6 +374,79 @@ static void adj2_tiles(const awefd_model *m, int *ntz2, int *ntx2)
     *ntx2 = (m->np[1] + sx - 1) / sx;
 }
 
+/* The tile of the resident adjoint loop, and its rim words: for the models
+ * whose forward loop is resident, the fewest rows per wave whose blocks fit
+ * one per CU.  rt.on = 0: the loop of one launch per step. */
+static void resadj_pick(awefd_model *m, adj_state *s)
+{
+    static const int list[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 0};
+    int cus = 0;
+    if (s->E.p) return;                        /* the grid's: picked before */
+    s->rt.on = 0;
+    if (!m->res.on || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev) != hipSuccess) return;
+    for (const int *rx = list; *rx; rx++) {
+        awefd__res_tile_of(m, m->nop, *rx, 1, &s->rt);
+        if (s->rt.on && (long)s->rt.ntz * s->rt.ntx <= cus) break;
+        s->rt.on = 0;
+    }
+    if (!s->rt.on) return;
+    const size_t bytes = sizeof(unsigned long long) * 2 * (size_t)s->rt.words * s->rt.ntz * s->rt.ntx;
+    s->tag = 1;
+    s->rt.on = awefd__resadj_blocks(m->nop, s->rt.rx) >= 1 && !awefd__res_grow(&s->E, bytes) &&
+               !awefd_launch_fill(s->E.p, (long)(bytes / sizeof(float)), 0.f, m->stream);
+}
+
+/* Every backward step of a run that kept its fields, as one launch; *done = 0:
+ * not taken, or given up on waiting for a block. */
+static int resadj_run(awefd_model *m, adj_state *s, const awefd_adj2d_args *g, int *done)
+{
+    awefd_resadj_args a;
+    int rc;
+    *done = 0;
+    if (!s->rt.on || !m->res.on) return AWEFD_OK;
+    memset(&a, 0, sizeof a);
+    a.nz = g->nz;
+    a.nx = g->nx;
+    a.ld = g->ld;
+    a.ntz = s->rt.ntz;
+    a.ntx = s->rt.ntx;
+    a.nt = m->p.nt;
+    a.c0f = s->ck;
+    a.seg = s->seg;
+    a.nal = m->nalloc;
+    a.V = g->V;
+    a.gV = g->gV;
+    a.sp1 = g->sp1;
+    a.sp2 = g->sp2;
+    a.c0 = g->c0;
+    for (int k = 0; k < m->nop; k++) {
+        a.cz[k] = g->cz[k];
+        a.cx[k] = g->cx[k];
+    }
+    a.rbeg = s->rbegr;
+    a.rinj = s->rinjr;
+    a.sbeg = s->sbegr;
+    a.sinj = s->sinjr;
+    a.res = g->res;
+    a.nr = g->nr;
+    a.wav = g->wav;
+    a.wstride = g->wstride;
+    a.E = (unsigned long long *)s->E.p;
+    a.stop = m->res.stop;
+    awefd__res_wait(&a.wmask, &a.wticks);
+    if ((rc = awefd__res_tags(&s->E, &s->tag, a.nt, m->stream, &a.tag0))) return rc;
+    if (awefd__resadj_launch(&a, a.ntz * a.ntx, m->nop, s->rt.rx, m->stream)) {
+        (void)hipGetLastError();               /* this device cannot hold the blocks */
+        s->rt.on = 0;
+        return AWEFD_OK;
+    }
+    const hipError_t e = hipStreamSynchronize(m->stream);
+    if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "resident adjoint: %s", hipGetErrorString(e));
+    *done = *(volatile unsigned *)m->res.stop == 0;
+    *m->res.stop = 0;
+    return AWEFD_OK;
+}
+
 /* Buffers and point buckets of the backward pass (kept across calls). */
 int awefd__adj_prepare(awefd_model *m)
 {
@@ -392,17 +477,26 @@ int awefd__adj_prepare(awefd_model *m)
         int ntz2, ntx2;
         adj2_tiles(m, &ntz2, &ntx2);
         const int ex = m->p.expl;
-        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz, ntx, tx, 0, &s->rinj, &s->rbeg))) return rc;
-        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz, ntx, tx, 0, &s->sinj, &s->sbeg))) return rc;
-        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz, ntxb, txb, 0, &s->rinjb, &s->rbegb))) return rc;
-        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz, ntxb, txb, 0, &s->sinjb, &s->sbegb)))
+        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz, ntx, 64, tx, 0, &s->rinj, &s->rbeg))) return rc;
+        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz, ntx, 64, tx, 0, &s->sinj, &s->sbeg))) return rc;
+        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz, ntxb, 64, txb, 0, &s->rinjb, &s->rbegb))) return rc;
+        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz, ntxb, 64, txb, 0, &s->sinjb, &s->sbegb)))
             return rc;
-        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz2, ntx2, AWEFD_ADJ2_ROWS, m->nop, &s->rinj2,
+        if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, ntz2, ntx2, 64, AWEFD_ADJ2_ROWS, m->nop, &s->rinj2,
                                 &s->rbeg2)))
             return rc;
-        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz2, ntx2, AWEFD_ADJ2_ROWS, m->nop, &s->sinj2,
+        if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz2, ntx2, 64, AWEFD_ADJ2_ROWS, m->nop, &s->sinj2,
                                 &s->sbeg2)))
             return rc;
+        resadj_pick(m, s);
+        if (s->rt.on) {
+            const awefd_res_tile *t = &s->rt;
+            const int nw = t->ntx * AWEFD_RES_NWAVE;
+            if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, t->ntz, nw, t->zw, t->rx, 0, &s->rinjr, &s->rbegr)))
+                return rc;
+            if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, t->ntz, nw, t->zw, t->rx, 0, &s->sinjr, &s->sbegr)))
+                return rc;
+        }
         s->lists_ok = 1;
         s->lists_gen = m->bgen;
     }
@@ -504,7 +598,9 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
     if ((rc = awefd__adj_prepare(m))) goto done;
     awefd__adj_args(m, d_res, &g);
     HIPCHK(hipMemcpy(s->d_args, &g, sizeof g, hipMemcpyHostToDevice));
-    {
+    int done = 0;
+    if (K == nt && (rc = resadj_run(m, s, &g, &done))) goto done;
+    if (!done) {
         awefd_copy_job z[3];
         awefd__adj_zero_jobs(m, z);
         for (int i = 0; i < 3; i++) {
@@ -518,7 +614,7 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
     /* recompute steps: out of place, no trace extraction */
     awefd__cart_args(m, &a);
     a.nr = 0;
-    for (int k = nck - 1; k >= 0; k--) {
+    for (int k = done ? -1 : nck - 1; k >= 0; k--) {
         const int n0 = k * K, n1 = n0 + K < nt ? n0 + K : nt;
         float *ckc = awefd__adj_ckpt(m, k), *ckp = ckc + m->nalloc;
 #define FIELD(n) ((n) == n0 ? ckc : s->seg + (size_t)((n) - n0 - 1) * m->nalloc)
