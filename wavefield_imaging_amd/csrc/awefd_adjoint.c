@@ -385,7 +385,7 @@ static void resadj_pick(awefd_model *m, adj_state *s)
     s->rt.on = 0;
     if (!m->res.on || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev) != hipSuccess) return;
     for (const int *rx = list; *rx; rx++) {
-        awefd__res_tile_of(m, m->nop, *rx, 1, &s->rt);
+        awefd__res_tile_of(m, m->nop, *rx, 1, AWEFD_RES_NWAVE, &s->rt);
         if (s->rt.on && (long)s->rt.ntz * s->rt.ntx <= cus) break;
         s->rt.on = 0;
     }
@@ -491,7 +491,7 @@ int awefd__adj_prepare(awefd_model *m)
         resadj_pick(m, s);
         if (s->rt.on) {
             const awefd_res_tile *t = &s->rt;
-            const int nw = t->ntx * AWEFD_RES_NWAVE;
+            const int nw = t->ntx * t->nw;
             if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, t->ntz, nw, t->zw, t->rx, 0, &s->rinjr, &s->rbegr)))
                 return rc;
             if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, t->ntz, nw, t->zw, t->rx, 0, &s->sinjr, &s->sbegr)))

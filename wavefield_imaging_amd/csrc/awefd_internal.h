@@ -141,21 +141,21 @@ typedef struct {
     const awefd_rx3 *rx3;
 } awefd_cart_args;
 
-/* The resident 2-D loop (res_loop.h): blocks of AWEFD_RES_NWAVE waves; S
- * steps per exchange; a tile owns 64 - 2 S nop z nodes of 8 rx - 2 (S - 1)
- * nop x rows (rx: rows a wave computes). */
+/* The resident 2-D loops (res_loop.h, res_polar.hip, res_adj.hip): blocks of
+ * nw waves; S steps per exchange; a tile owns 64 - 2 S nop z nodes of
+ * nw rx - 2 (S - 1) nop x rows (rx: rows a wave computes). */
 #define AWEFD_RES_NWAVE 8
+#define AWEFD_RES_NWAVE2 16      /* cartesian, two steps per exchange          */
 #define AWEFD_RES_MAXNOP 4       /* stencil half-widths compiled               */
 typedef struct {
     int on;                      /* a compiled tile whose blocks fit           */
-    int rx, S;
+    int rx, S, nw;
     int zw, ox, ntz, ntx;        /* owned nodes of a tile, tiles               */
     long words;                  /* 64-bit words of a block's rim              */
 } awefd_res_tile;
 typedef struct {
     int n1, n2, ld;              /* padded grid, row stride                    */
     int ntz, ntx;                /* tiles                                      */
-    int blk0;                    /* batched: first block of this shot          */
     int nb, dabc;
     float c0, cz[AWEFD_RES_MAXNOP], cx[AWEFD_RES_MAXNOP];
     float bz[AWEFD_RES_MAXNOP], bx[AWEFD_RES_MAXNOP];
@@ -189,16 +189,12 @@ typedef struct {
     long long wticks;
 } awefd_res_args;
 
-/* one shot (many NULL) or the shots of a block table, all steps, cooperative
+/* every step of one shot, cooperative
  * (res_nop1.hip ... res_nop4.hip); resident blocks per CU (0: not compiled) */
-int awefd__res_launch1(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
-                       int vd, void *stream);
-int awefd__res_launch2(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
-                       int vd, void *stream);
-int awefd__res_launch3(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
-                       int vd, void *stream);
-int awefd__res_launch4(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, int rx, int S,
-                       int vd, void *stream);
+int awefd__res_launch1(const awefd_res_args *a, int nblk, int rx, int S, int vd, void *stream);
+int awefd__res_launch2(const awefd_res_args *a, int nblk, int rx, int S, int vd, void *stream);
+int awefd__res_launch3(const awefd_res_args *a, int nblk, int rx, int S, int vd, void *stream);
+int awefd__res_launch4(const awefd_res_args *a, int nblk, int rx, int S, int vd, void *stream);
 int awefd__res_blocks1(int rx, int S, int vd);
 int awefd__res_blocks2(int rx, int S, int vd);
 int awefd__res_blocks3(int rx, int S, int vd);

@@ -136,8 +136,7 @@ int  awefd__cart_buckets(const awefd_model *m, int tz, int ntz, int tx, awefd_in
 /* resident 2-D loop (awefd_resident.c) */
 int  awefd__res_form(const awefd_model *m);
 void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t);
-int  awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *one, const awefd_res_args *many,
-                       const int *bshot, int nblk, int vd, hipStream_t s);
+int  awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *a, int nblk, int vd, hipStream_t s);
 int  awefd__res_blocks(int nop, const awefd_res_tile *t, int vd);
 int  awefd__res_create(awefd_model *m);
 void awefd__res_free(awefd_model *m);
@@ -150,7 +149,7 @@ void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_
                      const awefd_res_buf *rec, size_t idx_off, float *dtr, awefd_res_args *a);
 int  awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done);
 int  awefd__res_grow(awefd_res_buf *b, size_t bytes);
-void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_tile *t);
+void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, int nw, awefd_res_tile *t);
 int  awefd__res_buffers(awefd_model *m);
 void awefd__res_wait(unsigned *wmask, long long *wticks);
 int  awefd__res_finish(awefd_model *m, int launched, int *done);

@@ -49,7 +49,7 @@ int awefd__res_form(const awefd_model *m)
            !(e && atoi(e) == 0);
 }
 
-typedef int launch_fn(const awefd_res_args *, const awefd_res_args *, const int *, int, int, int, int, void *);
+typedef int launch_fn(const awefd_res_args *, int, int, int, int, void *);
 typedef int blocks_fn(int, int, int);
 static launch_fn *const LAUNCH[AWEFD_RES_MAXNOP] = {awefd__res_launch1, awefd__res_launch2, awefd__res_launch3,
                                                     awefd__res_launch4};
@@ -58,13 +58,14 @@ static blocks_fn *const BLOCKS[AWEFD_RES_MAXNOP] = {awefd__res_blocks1, awefd__r
 
 /* A tile of rx rows per wave and S steps per exchange on this grid, for a
  * stencil half-width nop. */
-void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_tile *t)
+void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, int nw, awefd_res_tile *t)
 {
     const int H = S * nop;
+    t->nw = nw;
     t->rx = rx;
     t->S = S;
     t->zw = 64 - 2 * H;
-    t->ox = AWEFD_RES_NWAVE * rx - 2 * (S - 1) * nop;
+    t->ox = nw * rx - 2 * (S - 1) * nop;
     t->on = t->ox >= H;
     t->ntz = (m->np[0] + t->zw - 1) / t->zw;
     t->ntx = t->on ? (m->np[1] + t->ox - 1) / t->ox : 0;
@@ -72,11 +73,11 @@ void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, awefd_res_
 }
 
 /* The compiled tile with the fewest rows per wave whose blocks fit nblk: two
- * steps per exchange up to 12 rows, above (the margin then costs more nodes
- * than the chip has) one. */
+ * steps per exchange up to 6 rows of 16 waves, above (the margin then costs
+ * more nodes than the chip has) one and 8 waves. */
 void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t)
 {
-    static const int rx2[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 0}, rx2v[] = {2, 3, 4, 6, 8, 0},
+    static const int rx2[] = {1, 2, 3, 4, 5, 6, 0}, rx2v[] = {1, 2, 3, 4, 0},
                      rx1[] = {8, 10, 12, 14, 16, 20, 24, 28, 32, 0};
     memset(t, 0, sizeof *t);
     const char *e = getenv("AWEFD_RES_STEPS");
@@ -84,17 +85,16 @@ void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t)
         const int *list = S == 1 ? (vd ? rx1 + 9 : rx1) : vd ? rx2v : rx2;
         if (e && atoi(e) != S) continue;
         for (; *list; list++) {
-            awefd__res_tile_of(m, m->nop, *list, S, t);
+            awefd__res_tile_of(m, m->nop, *list, S, S == 2 ? AWEFD_RES_NWAVE2 : AWEFD_RES_NWAVE, t);
             if (t->on && (long)t->ntz * t->ntx <= nblk) return;
         }
     }
     t->on = 0;
 }
 
-int awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *one, const awefd_res_args *many,
-                      const int *bshot, int nblk, int vd, hipStream_t s)
+int awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *a, int nblk, int vd, hipStream_t s)
 {
-    return LAUNCH[nop - 1](one, many, bshot, nblk, t->rx, t->S, vd, s);
+    return LAUNCH[nop - 1](a, nblk, t->rx, t->S, vd, s);
 }
 
 int awefd__res_blocks(int nop, const awefd_res_tile *t, int vd)
@@ -115,8 +115,8 @@ int awefd__res_buffers(awefd_model *m)
     r->tag = 1;
     r->on = 1;
     if (getenv("AWEFD_VERBOSE"))
-        fprintf(stderr, "awefd: resident 2-D loop: %d x %d blocks, %d rows per wave, %d steps per exchange\n", r->t.ntz,
-                r->t.ntx, r->t.rx, r->t.S);
+        fprintf(stderr, "awefd: resident 2-D loop: %d x %d blocks of %d waves, %d rows per wave, %d steps per exchange\n",
+                r->t.ntz, r->t.ntx, r->t.nw, r->t.rx, r->t.S);
     return AWEFD_OK;
 }
 
@@ -158,7 +158,7 @@ int awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *o
     long n;
     int rc = awefd__cart_buckets(m, m->np[0], 1, m->np[1], &e, &one, &nbucket, &n);
     if (rc) return rc;
-    const int ext = (t->S - 1) * m->nop, nb = t->ntz * t->ntx * AWEFD_RES_NWAVE;
+    const int ext = (t->S - 1) * m->nop, nb = t->ntz * t->ntx * t->nw;
     const size_t head = (sizeof(int) * (size_t)(nb + 1) + 15) / 16 * 16;
     char *h = NULL;
     for (int pass = 0; pass < 2 && !rc; pass++) {
@@ -169,8 +169,8 @@ int awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *o
             for (int bx = (e[i].x - ext > 0 ? (e[i].x - ext) / t->ox : 0); bx <= (e[i].x + ext) / t->ox && bx < t->ntx; bx++)
                 for (int bz = (e[i].z - ext > 0 ? (e[i].z - ext) / t->zw : 0); bz <= (e[i].z + ext) / t->zw && bz < t->ntz; bz++) {
                     const int lr = e[i].x - (bx * t->ox - ext);
-                    if (lr < 0 || lr >= AWEFD_RES_NWAVE * t->rx) continue;
-                    const int b = (bz + t->ntz * bx) * AWEFD_RES_NWAVE + lr / t->rx;
+                    if (lr < 0 || lr >= t->nw * t->rx) continue;
+                    const int b = (bz + t->ntz * bx) * t->nw + lr / t->rx;
                     if (pass == 0) cnt[b + 1]++;
                     else ((awefd_inj *)(h + head))[beg[b]++] = e[i];
                 }
@@ -336,6 +336,6 @@ int awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done)
     a.stop = r->stop;
     int rc = awefd__res_tags(&r->E, &r->tag, a.nt, m->stream, &a.tag0);
     if (rc) return rc;
-    return awefd__res_finish(m, awefd__res_launch(m->nop, &r->t, &a, NULL, NULL, r->t.ntz * r->t.ntx, vd, m->stream),
+    return awefd__res_finish(m, awefd__res_launch(m->nop, &r->t, &a, r->t.ntz * r->t.ntx, vd, m->stream),
                              done);
 }

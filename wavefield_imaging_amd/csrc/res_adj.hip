@@ -21,10 +21,10 @@
 namespace {
 
 template <int NOP, int RX>
-__global__ __launch_bounds__(NTHR) void k_adj_res(const awefd_resadj_args a)
+__global__ __launch_bounds__(AWEFD_RES_NWAVE * WAVE) void k_adj_res(const awefd_resadj_args a)
 {
     using T = tile<NOP, RX, 1>;
-    constexpr int H = T::H, ZW = T::ZW, OX = T::OX, ISH = T::ISH, R = RX + 2 * NOP;
+    constexpr int NTHR = T::NTHR, H = T::H, ZW = T::ZW, OX = T::OX, ISH = T::ISH, R = RX + 2 * NOP;
     extern __shared__ float img[];                     /* [2][rows + 2 NOP][64] */
     __shared__ int s_stop[2];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_res(const awefd_resadj_args a)
 
     /* receiver and source entries of this wave's rows, the first 64 one per
      * lane with their amplitudes of the coming step */
-    const int col = tz + a.ntz * (txi * NW + wv);
+    const int col = tz + a.ntz * (txi * AWEFD_RES_NWAVE + wv);
     const int rb = a.rbeg[col], rn = a.rbeg[col + 1] - rb, sb = a.sbeg[col], sn = a.sbeg[col + 1] - sb;
     int rz = 0, rx = 0, rs = 0, sz = 0, sx = 0, ss = 0;
     float rw = 0.f, sw = 0.f;
@@ -205,6 +205,7 @@ __global__ __launch_bounds__(NTHR) void k_adj_res(const awefd_resadj_args a)
 
 template <int NOP, int RX>
 struct kernel {
+    static constexpr int NTHR = AWEFD_RES_NWAVE * WAVE;
     static constexpr size_t LDS = sizeof(float) * 2 * (size_t)tile<NOP, RX, 1>::ISH;
 
     static hipError_t attr()

@@ -38,14 +38,18 @@
  * the host then runs the one-launch-per-step loop instead.
  *
  * Tile.  A wave holds 64 z lanes, the outer S NOP on each side the margin,
- * of RX x rows; 8 waves a block.  z neighbours are DPP shifts inside the
+ * of RX x rows; 16 waves a block with S = 2 (4 per SIMD, up to 96 rows: the
+ * waves' chains of dependent steps overlap; 8 waves of twice the rows took
+ * 1.47 us a step for 140 x 240 nodes against 1.24, 1.49 against 1.30 for
+ * 500 x 900, 2.5 against 2.3 for 800 x 1500), 8 with S = 1, whose rows need
+ * the registers (28 rows as 16 waves of 14: 13.4 us against 9.5).  z neighbours are DPP shifts inside the
  * wave, x neighbours rows of the block's LDS image, which also feeds the
  * trace extraction (a receiver belongs to the block of its first corner; the
  * other corners are in the margin).  The image is double-buffered by the
  * parity of the step.
  *
- * Measured per step, against one launch per step: 140 x 240 nodes 1.19 us
- * (3.1 as a graph), 500 x 900 1.41 us (4.7 launched, 3.66 as a graph), 1101 x
+ * Measured per step, against one launch per step: 140 x 240 nodes 1.24 us
+ * (3.1 as a graph), 500 x 900 1.30 us (4.7 launched, 3.66 as a graph), 1101 x
  * 2877 with nop 4 9.2 us (11.2).  What a step takes at the small sizes: the
  * exchange 0.6 us per step with S = 2 (1.0 with S = 1: 2.3 and 2.0 us in
  * all), barriers and LDS rows 0.3, arithmetic 0.1-0.3; at 28 rows per wave
@@ -161,21 +165,22 @@ __device__ __forceinline__ void rows(const float (&c)[RX + 2 * NOP], float (&p)[
     }
 }
 
+/* two steps per exchange: 16 waves a block */
+constexpr int nwave(int S) { return S == 2 ? AWEFD_RES_NWAVE2 : AWEFD_RES_NWAVE; }
+
 template <int NOP, int RX, int S, bool VD>
-__global__ __launch_bounds__(NTHR) void k_cart2d_res(const awefd_res_args, const awefd_res_args *many,
-                                                     const int *bshot)
+__global__ __launch_bounds__(nwave(S) * WAVE) void k_cart2d_res(const awefd_res_args)
 {
-    using T = tile<NOP, RX, S>;
-    constexpr int H = T::H, EXT = T::EXT, ZW = T::ZW, OX = T::OX, ISH = T::ISH;
+    constexpr int NW = nwave(S);
+    using T = tile<NOP, RX, S, NW>;
+    constexpr int NTHR = T::NTHR, H = T::H, EXT = T::EXT, ZW = T::ZW, OX = T::OX, ISH = T::ISH;
     extern __shared__ float img[];                     /* [2][rows + 2 NOP][64] */
     __shared__ int s_stop[2];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    /* this shot's arguments, in constant memory either way (the kernel's own
-     * argument block, or the batch's table) */
-    const cargs &a = many ? ((const cargs *)(uintptr_t)many)[bshot[blockIdx.x]]
-                          : *(const cargs *)__builtin_amdgcn_kernarg_segment_ptr();
-    const int lb = many ? (int)blockIdx.x - a.blk0 : xcd_remap(blockIdx.x, a.ntz * a.ntx);
+    /* the arguments in constant memory (the kernel's own block) */
+    const cargs &a = *(const cargs *)__builtin_amdgcn_kernarg_segment_ptr();
+    const int lb = xcd_remap(blockIdx.x, a.ntz * a.ntx);
     const int tz = lb % a.ntz, txi = lb / a.ntz;
     const int n1 = a.n1, n2 = a.n2;
     const int z0 = tz * ZW - H, xb = txi * OX - H;     /* node of lane 0 and of image row 0 */
@@ -405,7 +410,8 @@ __global__ __launch_bounds__(NTHR) void k_cart2d_res(const awefd_res_args, const
 
 template <int NOP, int RX, int S, bool VD>
 struct kernel {
-    static constexpr size_t LDS = sizeof(float) * 2 * (size_t)tile<NOP, RX, S>::ISH;
+    static constexpr size_t LDS = sizeof(float) * 2 * (size_t)tile<NOP, RX, S, nwave(S)>::ISH;
+    static constexpr int NTHR = nwave(S) * WAVE;
 
     static hipError_t attr()
     {
@@ -413,12 +419,12 @@ struct kernel {
         return hipFuncSetAttribute((const void *)k_cart2d_res<NOP, RX, S, VD>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS);
     }
-    static int launch(const awefd_res_args *one, const awefd_res_args *many, const int *bshot, int nblk, hipStream_t s)
+    static int launch(const awefd_res_args *one, int nblk, hipStream_t s)
     {
         const hipError_t e = attr();
         if (e != hipSuccess) return (int)e;
         awefd_res_args a = *one;
-        void *args[] = {&a, &many, &bshot};
+        void *args[] = {&a};
         return (int)hipLaunchCooperativeKernel((const void *)k_cart2d_res<NOP, RX, S, VD>, dim3(nblk), dim3(NTHR), args,
                                                (unsigned)LDS, s);
     }
@@ -439,11 +445,11 @@ int pick(int rx, int S, int vd, F f)
 {
 #define RX_CASE(n, s, v) case n: return f(kernel<NOP, n, s, v>());
     if (S == 2 && vd) switch (rx) {
-        RX_CASE(2, 2, true) RX_CASE(3, 2, true) RX_CASE(4, 2, true) RX_CASE(6, 2, true) RX_CASE(8, 2, true)
+        RX_CASE(1, 2, true) RX_CASE(2, 2, true) RX_CASE(3, 2, true) RX_CASE(4, 2, true)
     }
     if (S == 2 && !vd) switch (rx) {
-        RX_CASE(2, 2, false) RX_CASE(3, 2, false) RX_CASE(4, 2, false) RX_CASE(5, 2, false) RX_CASE(6, 2, false)
-        RX_CASE(7, 2, false) RX_CASE(8, 2, false) RX_CASE(10, 2, false) RX_CASE(12, 2, false)
+        RX_CASE(1, 2, false) RX_CASE(2, 2, false) RX_CASE(3, 2, false) RX_CASE(4, 2, false) RX_CASE(5, 2, false)
+        RX_CASE(6, 2, false)
     }
     if (S == 1 && !vd) switch (rx) {
         RX_CASE(8, 1, false) RX_CASE(10, 1, false) RX_CASE(12, 1, false) RX_CASE(14, 1, false) RX_CASE(16, 1, false)
@@ -458,10 +464,9 @@ int pick(int rx, int S, int vd, F f)
 #define RES_CAT2(a, b) a##b
 #define RES_CAT(a, b) RES_CAT2(a, b)
 
-extern "C" int RES_CAT(awefd__res_launch, RES_NOP)(const awefd_res_args *one, const awefd_res_args *many,
-                                                   const int *bshot, int nblk, int rx, int S, int vd, void *stream)
+extern "C" int RES_CAT(awefd__res_launch, RES_NOP)(const awefd_res_args *a, int nblk, int rx, int S, int vd, void *stream)
 {
-    const int e = pick<RES_NOP>(rx, S, vd, [&](auto k) { return k.launch(one, many, bshot, nblk, (hipStream_t)stream); });
+    const int e = pick<RES_NOP>(rx, S, vd, [&](auto k) { return k.launch(a, nblk, (hipStream_t)stream); });
     return e < 0 ? (int)hipErrorInvalidValue : e;
 }
 

@@ -46,10 +46,10 @@ __device__ __forceinline__ int depth(int ir, int ith, int n1, int n2, int nb)
 }
 
 template <int RX, int S>
-__global__ __launch_bounds__(NTHR) void k_polar_res(const awefd_polar_args a)
+__global__ __launch_bounds__(AWEFD_RES_NWAVE * WAVE) void k_polar_res(const awefd_polar_args a)
 {
     using T = tile<1, RX, S>;
-    constexpr int H = T::H, EXT = T::EXT, ZW = T::ZW, OX = T::OX, ISH = T::ISH, MI = AWEFD_POLAR_ITEMS / NTHR;
+    constexpr int NTHR = T::NTHR, H = T::H, EXT = T::EXT, ZW = T::ZW, OX = T::OX, ISH = T::ISH, MI = AWEFD_POLAR_ITEMS / NTHR;
     extern __shared__ float img[];                     /* [2][rows + 2][64] */
     __shared__ int s_stop[2];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -321,6 +321,7 @@ __global__ __launch_bounds__(NTHR) void k_polar_res(const awefd_polar_args a)
 
 template <int RX, int S>
 struct kernel {
+    static constexpr int NTHR = AWEFD_RES_NWAVE * WAVE;
     static constexpr size_t LDS = sizeof(float) * 2 * (size_t)tile<1, RX, S>::ISH;
 
     static hipError_t attr()

@@ -13,8 +13,6 @@
 namespace {
 
 using namespace awefd;
-constexpr int NW = AWEFD_RES_NWAVE;
-constexpr int NTHR = NW * WAVE;
 
 typedef unsigned long long u64;
 __device__ __forceinline__ void put_word(u64 *p, unsigned tag, float v)
@@ -42,9 +40,10 @@ __device__ __forceinline__ float dn1(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
 }
 
-/* The tile and its margin. */
-template <int NOP, int RX, int S>
+/* The tile and its margin; NW: waves of its block. */
+template <int NOP, int RX, int S, int NW = AWEFD_RES_NWAVE>
 struct tile {
+    static constexpr int NTHR = NW * WAVE;
     static constexpr int H = S * NOP;                  /* margin of the image   */
     static constexpr int EXT = (S - 1) * NOP;          /* ... that is computed  */
     static constexpr int ZW = WAVE - 2 * H;            /* owned z lanes         */
@@ -83,7 +82,7 @@ struct exchange {
         constexpr int H = T::H, ZW = T::ZW, K = T::K, W = T::WORDS;
 #pragma unroll
         for (int i = 0; i < MP; i++) {
-            const int w = tid + i * NTHR;
+            const int w = tid + i * T::NTHR;
             int at = -1;
             if (w < T::NZ) at = (H + w / H) * WAVE + H + w % H;
             else if (w >= T::ZH && w < T::ZH + T::NZ) at = (H + (w - T::ZH) / H) * WAVE + WAVE - 2 * H + (w - T::ZH) % H;
@@ -96,7 +95,7 @@ struct exchange {
         const bool lz = tz > 0, hz = tz + 1 < ntz, lx = txi > 0, hx = txi + 1 < ntx;
 #pragma unroll
         for (int i = 0; i < MW; i++) {
-            int w = tid + i * NTHR, s = -1;
+            int w = tid + i * T::NTHR, s = -1;
             dst[i] = 0;
             if (w < T::NZ) {                           /* z below: lanes 0..H-1 */
                 if (lz) s = (b - 1) * W + T::ZH + w;

@@ -667,7 +667,7 @@ static int polar_create(awefd_model *m)
     for (int S = 2; S >= 1; S--) {
         if (st && atoi(st) != S) continue;
         for (const int *rx = S == 2 ? rx2 : rx1; *rx; rx++) {
-            awefd__res_tile_of(m, 1, *rx, S, &r->t);
+            awefd__res_tile_of(m, 1, *rx, S, AWEFD_RES_NWAVE, &r->t);
             const awefd_res_tile *t = &r->t;
             const int lz = m->np[0] - (t->ntz - 1) * t->zw, lx = m->np[1] - (t->ntx - 1) * t->ox;
             size_t off, bytes;
