@@ -18,8 +18,8 @@ def test_smallest_grids(orc, fdorder, n2, n3):
     par = dict(n=n, o=[0.0] * 3, d=[5.0] * 3, nt=25, dt=synth.DT, nb=nb, dabc=True, fdorder=fdorder, expl=False)
     vel = rng.uniform(1.2e8, 3.0e8, n[::-1]).astype(np.float32)
     lo, hi = -5.0 * nb, np.array([n2, n3, n[0]]) * 5.0 + 5.0 * nb - 8.0
-    pts = rng.uniform(lo, hi, (12, 3)).astype(np.float32)
-    wav = rng.standard_normal((25, 12)).astype(np.float32)
+    pts = rng.uniform(lo, hi, (200, 3)).astype(np.float32)
+    wav = rng.standard_normal((25, 200)).astype(np.float32)
     tr, _, f = awefd.run("cart3d", par, vel, pts, pts, wav)
     ref, uf, _ = orc.run("cart3d", par, vel, pts, pts, wav)
     assert np.any(f)
