@@ -123,3 +123,9 @@ def test_a_block_that_gives_up(monkeypatch):
     got = awefd.run("cart2d", par, vel, sou, rec, wav)
     np.testing.assert_array_equal(got[0], want[0])
     np.testing.assert_array_equal(got[2], want[2])
+
+
+# 18, 26 and 30 rows per wave at fdorder 4, and 30 at fdorder 8
+@pytest.mark.parametrize("n1,n2,fdorder", [(1000, 2100, 4), (1000, 3050, 4), (1000, 3500, 4), (1001, 2777, 8)])
+def test_even_row_counts(n1, n2, fdorder, monkeypatch, capfd):
+    _both(_case(n1, n2, 10, 8, 29, nsrc=40, fdorder=fdorder), monkeypatch, capfd)

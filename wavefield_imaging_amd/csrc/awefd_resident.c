@@ -78,11 +78,11 @@ void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, int nw, aw
 void awefd__res_pick(const awefd_model *m, int vd, int nblk, awefd_res_tile *t)
 {
     static const int rx2[] = {1, 2, 3, 4, 5, 6, 0}, rx2v[] = {1, 2, 3, 4, 0},
-                     rx1[] = {8, 10, 12, 14, 16, 20, 24, 28, 32, 0};
+                     rx1[] = {8, 10, 12, 14, 16, 18, 20, 22, 24, 26, 28, 30, 32, 0};
     memset(t, 0, sizeof *t);
     const char *e = getenv("AWEFD_RES_STEPS");
     for (int S = 2; S >= 1; S--) {
-        const int *list = S == 1 ? (vd ? rx1 + 9 : rx1) : vd ? rx2v : rx2;
+        const int *list = S == 1 ? (vd ? rx1 + 13 : rx1) : vd ? rx2v : rx2;
         if (e && atoi(e) != S) continue;
         for (; *list; list++) {
             awefd__res_tile_of(m, m->nop, *list, S, S == 2 ? AWEFD_RES_NWAVE2 : AWEFD_RES_NWAVE, t);

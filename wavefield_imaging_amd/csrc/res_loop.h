@@ -50,10 +50,11 @@
  *
  * Measured per step, against one launch per step: 140 x 240 nodes 1.24 us
  * (3.1 as a graph), 500 x 900 1.30 us (4.7 launched, 3.66 as a graph), 1101 x
- * 2877 with nop 4 9.2 us (11.2).  What a step takes at the small sizes: the
+ * 2877 with nop 4 8.2 us (11.2).  What a step takes at the small sizes: the
  * exchange 0.6 us per step with S = 2 (1.0 with S = 1: 2.3 and 2.0 us in
- * all), barriers and LDS rows 0.3, arithmetic 0.1-0.3; at 28 rows per wave
- * the arithmetic 4 us and the exchange of 2,500 words a block 3.5.
+ * all), barriers and LDS rows 0.3, arithmetic 0.1-0.3; at 30 rows per wave
+ * the arithmetic about 4 us and the exchange of 2,300 words a block 3.5 (the
+ * even row counts matter there: 32 rows of which 30 were needed took 9.4).
  *
  * Arithmetic, order and selections are cart_step_body's (cart_kernels.hip)
  * node for node, lazy second sponge included: the same bits.
@@ -453,7 +454,8 @@ int pick(int rx, int S, int vd, F f)
     }
     if (S == 1 && !vd) switch (rx) {
         RX_CASE(8, 1, false) RX_CASE(10, 1, false) RX_CASE(12, 1, false) RX_CASE(14, 1, false) RX_CASE(16, 1, false)
-        RX_CASE(20, 1, false) RX_CASE(24, 1, false) RX_CASE(28, 1, false) RX_CASE(32, 1, false)
+        RX_CASE(18, 1, false) RX_CASE(20, 1, false) RX_CASE(22, 1, false) RX_CASE(24, 1, false) RX_CASE(26, 1, false)
+        RX_CASE(28, 1, false) RX_CASE(30, 1, false) RX_CASE(32, 1, false)
     }
 #undef RX_CASE
     return -1;
