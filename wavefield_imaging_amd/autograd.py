@@ -5,8 +5,8 @@ slowness, for torch.
 a squared-slowness tensor (shape (n2, n1), n1 fastest, float32, on the
 model's GPU) to the (nt, nr) trace tensor of the same loop as sfAWEFDcart2D
 (MAWEFDcart2Dcpu.c:297-383).  The forward pass keeps a checkpoint of the
-field pair every ``ckpt`` steps (0: every field while
-three quarters of the card's memory stay free, else ceil(sqrt(nt))); ``backward`` runs the
+field pair every ``ckpt`` steps (0: every field while three quarters of the
+card's memory stay free, else ceil(sqrt(nt))); ``backward`` runs the
 hand-written adjoint kernels from those checkpoints (awefd_adjoint_grad in
 the C ABI), so ``loss.backward()`` gives dloss/dslow for any loss of the
 traces.  The reference has no gradient; this layer has no counterpart there.
