@@ -1,0 +1,98 @@
+"""The host code's own paths, on the CPU: the C sources against a HIP runtime
+without a GPU (hip_stub.c), which can refuse an allocation, return a launch
+error or let a resident loop give up."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from wavefield_imaging_amd import _lib as L
+from wavefield_imaging_amd import awefd
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(ROOT, "wavefield_imaging_amd", "csrc")
+HOST = ("awefd_api.c", "awefd_setup.c", "spher_host.c", "awefd_batch.c", "awefd_adjoint.c", "awefd_resident.c")
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "libhost.so")
+    subprocess.run(["gcc", "-O1", "-g", "-shared", "-fPIC", "-std=gnu99", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+                    "-Wl,-Bsymbolic", "-I", SRC, "-I", os.path.join(ROOT, "include"), "-I", "/opt/rocm/include",
+                    "-o", so] + [os.path.join(SRC, f) for f in HOST] + [os.path.join(ROOT, "tests", "hip_stub.c")]
+                   + ["-lm", "-lpthread"], check=True)
+    return so
+
+
+class Stub:
+    def __init__(self, lib):
+        self.lib = lib
+
+    def reset(self, fail_at=0, fail_above=0):
+        self.lib.stub_reset(C.c_long(fail_at), C.c_size_t(fail_above))
+
+    def get(self, name):
+        return C.c_long.in_dll(self.lib, "stub_" + name).value
+
+    def set(self, name, v):
+        (C.c_long if name == "fail_at" else C.c_int).in_dll(self.lib, "stub_" + name).value = v
+
+
+@pytest.fixture
+def stub(built, monkeypatch):
+    """The binding on the stubbed library for the time of one test."""
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L, "LIB_PATH", built)
+    for k in ("AWEFD_RESIDENT", "AWEFD_RES_STEPS", "AWEFD_RES_WAIT", "AWEFD_NARROW"):
+        monkeypatch.delenv(k, raising=False)
+    s = Stub(L.load())
+    s.reset()
+    yield s
+    s.reset()
+
+
+def _model(nt=9, n=(30, 40), nb=4, kind="cart2d", nr=5, **kw):
+    par = dict(n=list(n), o=[0.0, 0.0] if kind == "cart2d" else [3387.5e3, 0.785], d=[5.0, 5.0], nt=nt, dt=6.67e-9,
+               nb=nb, expl=True)
+    if kind == "spher2d":
+        par["d"] = [5.0, 5.0 / 3388.5e3]
+    par.update(kw)
+    m = awefd.Model(kind, par)
+    m.set_model(np.full(n[::-1], 1.7e8, np.float32))
+    x = np.array([par["o"][i] + 3.0 * par["d"][i] for i in ((1, 0) if kind == "cart2d" else (0, 1))], np.float32)
+    m.set_sources(x[None])
+    m.set_receivers(np.repeat(x[None], nr, 0))
+    m.set_wavelet(np.ones(nt, np.float32))
+    return m
+
+
+def _dev(*shape):
+    """An array of the stub's device memory, which is host memory."""
+    a = np.zeros(shape, np.float32)
+    return a, a.ctypes.data
+
+
+def _grad(m, ckpt, tr=None):
+    """A checkpointed run and its gradient."""
+    res, rp = _dev(m.nt, m.nr)
+    g, gp = _dev(m.params.n[1], m.params.n[0])
+    L.check(m.lib.awefd_run_ckpt(m.h, tr, ckpt))
+    L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
+
+
+def test_refused_fields_of_every_step_leave_no_error(stub):
+    """A gradient whose nt fields are refused takes ceil(sqrt(nt)) checkpoints
+    instead; the refused allocation's error must not be reported by the
+    launches that follow."""
+    with _model(nt=100) as m:
+        stub.reset(fail_above=60 * 4 * 64 * 48)      # 100 fields of 64 x 48 are, 20 and 10 are not
+        _grad(m, 0)
+    stub.reset()
+    with _model(nt=100) as m:                        # nor after an error that a caller has seen
+        stub.reset(fail_at=1)
+        with pytest.raises(L.AwefdError, match="out of memory"):
+            m.run()                                  # the trace buffer
+        stub.set("fail_at", 0)
+        m.run()

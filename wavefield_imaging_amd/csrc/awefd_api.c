@@ -23,12 +23,17 @@
 
 static __thread char g_err[512];
 
+/* The error is reported here, once: HIP keeps a failed call's code as the
+ * thread's last error until somebody takes it, and the launchers return the
+ * last error, so an allocation that failed and was worked around would fail
+ * the next launch. */
 int awefd__fail(int code, const char *fmt, ...)
 {
     va_list ap;
     va_start(ap, fmt);
     vsnprintf(g_err, sizeof g_err, fmt, ap);
     va_end(ap);
+    if (code == AWEFD_EHIP || code == AWEFD_ENOMEM) (void)hipGetLastError();
     return code;
 }
 
