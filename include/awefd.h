@@ -226,9 +226,12 @@ int awefd_batch_adjoint_grad(awefd_batch *b, const float *const *d_res, float *d
 /* The forward loop of awefd_run_dev (same traces, same final fields) that
  * also keeps the field pair of every ckpt-th step in device memory for
  * awefd_adjoint_grad: 2 ceil(nt/ckpt) padded fields.  With ckpt >= nt it keeps
- * every field (nt + 1 padded ones) and nothing is recomputed; ckpt <= 0 does
- * so while three quarters of the card's memory stay free, else takes
- * ceil(sqrt(nt)).  The gradient's bits do not depend on ckpt.
+ * every field (nt + 1 padded ones) and nothing is recomputed, if the device has
+ * memory for them (else the first pair, from which the gradient recomputes);
+ * ckpt <= 0 does so while three quarters of the card's memory stay free, else
+ * takes ceil(sqrt(nt)).  The fields stay with the handle until it is destroyed,
+ * until awefd_adjoint_release or until a run with another interval.  The
+ * gradient's bits do not depend on ckpt.
  * AWEFD_CART2D with constant density only. */
 int awefd_run_ckpt(awefd_model *m, float *d_traces, int ckpt);
 /* dJ/ds at the model of the last awefd_run_ckpt (AWEFD_ESTATE if a setter

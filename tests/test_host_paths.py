@@ -96,3 +96,70 @@ def test_refused_fields_of_every_step_leave_no_error(stub):
             m.run()                                  # the trace buffer
         stub.set("fail_at", 0)
         m.run()
+
+
+ALL = 60 * 4 * 64 * 48       # more than 60 padded fields of the default grid at once
+
+
+def test_an_interval_of_every_step_without_memory_for_it(stub):
+    """ckpt >= nt where the fields do not fit: the run keeps its one pair, as
+    with any interval, the gradient asks for its segment, and gives it by
+    recomputing once there is memory."""
+    with _model(nt=100) as m:
+        for ckpt in (100, 300):
+            stub.reset(fail_above=ALL)
+            L.check(m.lib.awefd_run_ckpt(m.h, None, ckpt))
+            assert stub.get("steps") == 100
+            res, rp = _dev(m.nt, m.nr)
+            g, gp = _dev(40, 30)
+            assert m.lib.awefd_adjoint_grad(m.h, rp, gp) == -3
+            assert b"gradient buffers" in m.lib.awefd_last_error()
+            stub.reset()
+            L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
+            assert stub.get("steps") == 99           # the segment's recomputed fields
+            assert stub.get("adjoint") == 0
+            m.lib.awefd_adjoint_release(m.h)
+        L.check(m.lib.awefd_run_ckpt(m.h, None, 100))
+        stub.reset()
+        L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
+        assert stub.get("steps") == 0 and stub.get("adjoint") == 1
+
+
+def test_a_batch_that_keeps_every_step_of_some_shots_only(stub):
+    ms = [_model(nt=30) for _ in range(2)]
+    b = awefd.Batch(ms)
+    res, rp = _dev(30, 5)
+    g, gp = _dev(40, 30)
+    stub.reset(fail_at=4)                            # the second shot's fields
+    b.run_ckpt(30)
+    assert stub.get("rows") == 0 and stub.get("recomputed") == 0
+    stub.reset()
+    b.adjoint_grad([rp, rp], gp)
+    assert stub.get("recomputed") == 2 * 29 or stub.get("recomputed") == 29     # one launch advances both shots
+    L.check(ms[0].lib.awefd_adjoint_grad(ms[0].h, rp, gp))
+    assert stub.get("adjoint") == 0                  # its fields were not kept either
+    stub.reset()
+    b.run_ckpt(30)
+    assert stub.get("rows") == 2 * 30
+    stub.reset()
+    b.adjoint_grad([rp, rp], gp)
+    assert stub.get("recomputed") == 0
+    # a default interval drops to checkpoints for every shot
+    for m in ms:
+        m.lib.awefd_adjoint_release(m.h)
+    stub.reset(fail_at=4)
+    b.run_ckpt(0)
+    stub.reset()
+    b.adjoint_grad([rp, rp], gp)
+    assert 0 < stub.get("recomputed") < 30
+    b.run_ckpt(30)
+    # a shot that was run on its own without its fields does not serve a batch that kept them
+    ms[1].lib.awefd_adjoint_release(ms[1].h)
+    stub.reset(fail_at=2)
+    L.check(ms[1].lib.awefd_run_ckpt(ms[1].h, None, 30))
+    stub.reset()
+    with pytest.raises(L.AwefdError, match="awefd_batch_run_ckpt"):
+        b.adjoint_grad([rp, rp], gp)
+    b.close()
+    for m in ms:
+        m.close()

@@ -37,6 +37,7 @@
 
 typedef struct {
     int K, nck, nt;
+    int kept;                 /* K = nt and the run stores every field    */
     unsigned gen;             /* model generation of the checkpoints      */
     int valid;
     float *ck;                /* nck pairs (c_{kK}, c_{kK-1})             */
@@ -227,11 +228,24 @@ int awefd__adj_ckpt_setup(awefd_model *m, int ckpt)
         s->K = K;
         s->nck = nck;
     }
+    s->kept = 0;
     if ((rc = dev_alloc(&s->ck, sizeof(float) * (size_t)m->nalloc * 2 * nck))) return rc;
-    /* one segment: the forward run stores its fields */
-    if (K < nt || K == 1 || !(rc = dev_alloc(&s->seg, sizeof(float) * (size_t)m->nalloc * (K - 1)))) return AWEFD_OK;
+    /* one segment: the forward run stores its fields, if there is memory */
+    s->kept = K == nt && (K == 1 || !dev_alloc(&s->seg, sizeof(float) * (size_t)m->nalloc * (K - 1)));
     const int few = (int)ceil(sqrt((double)nt));
-    return ckpt > 0 || few == nt ? rc : awefd__adj_ckpt_setup(m, few);
+    return s->kept || ckpt > 0 || K < nt || few == nt ? AWEFD_OK : awefd__adj_ckpt_setup(m, few);
+}
+
+/* Whether the run set up stores every field; a batch sets it for all its
+ * shots together. */
+int awefd__adj_kept(const awefd_model *m)
+{
+    return state(m) && state(m)->kept;
+}
+
+void awefd__adj_keep(awefd_model *m, int kept)
+{
+    state(m)->kept = kept;
 }
 
 /* Field n of a run that keeps them all; n = -1: the one before the first. */
@@ -333,7 +347,7 @@ int awefd_run_ckpt(awefd_model *m, float *d_traces, int ckpt)
     const size_t fb = sizeof(float) * (size_t)m->nalloc;
     awefd_cart_args a;
     if ((rc = awefd__ensure_traces(m))) goto done;
-    if (K == nt) {
+    if (s->kept) {
         if (!(rc = run_kept(m, d_traces ? d_traces : m->d_traces))) awefd__adj_mark(m);
         goto done;
     }
@@ -599,7 +613,7 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
     awefd__adj_args(m, d_res, &g);
     HIPCHK(hipMemcpy(s->d_args, &g, sizeof g, hipMemcpyHostToDevice));
     int done = 0;
-    if (K == nt && (rc = resadj_run(m, s, &g, &done))) goto done;
+    if (s->kept && (rc = resadj_run(m, s, &g, &done))) goto done;
     if (!done) {
         awefd_copy_job z[3];
         awefd__adj_zero_jobs(m, z);
@@ -618,7 +632,7 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
         const int n0 = k * K, n1 = n0 + K < nt ? n0 + K : nt;
         float *ckc = awefd__adj_ckpt(m, k), *ckp = ckc + m->nalloc;
 #define FIELD(n) ((n) == n0 ? ckc : s->seg + (size_t)((n) - n0 - 1) * m->nalloc)
-        for (int n = n0; n + 1 < n1 && K < nt; n++) {
+        for (int n = n0; n + 1 < n1 && !s->kept; n++) {
             a.C = FIELD(n);
             a.P = n == n0 ? ckp : FIELD(n - 1);
             a.Pn = FIELD(n + 1);

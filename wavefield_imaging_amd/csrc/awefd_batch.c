@@ -71,7 +71,7 @@ struct awefd_batch {
     awefd_cart_args *h;              /* host copy of d_shots                     */
     /* gradient: checkpointed forward and backward pass (awefd_adjoint.c holds
      * each shot's buffers) */
-    int K, nck;
+    int K, nck, kept;                /* kept: K = nt, every field stored         */
     awefd_copy_job *d_jobs;          /* checkpoint copies per (group, k)         */
     long *d_cbeg;
     long *joff, *jnch;               /* per (group, k): first job, chunks        */
@@ -1188,24 +1188,34 @@ static int run_kept(awefd_batch *b)
     return AWEFD_OK;
 }
 
+/* Checkpoint memory of every shot; *kept: all of them store every field. */
+static int ckpt_setup(awefd_batch *b, int ckpt, int *kept)
+{
+    int rc;
+    *kept = 1;
+    for (int s = 0; s < b->nshot; s++) {
+        if ((rc = awefd__adj_ckpt_setup(b->m[s], ckpt))) return rc;
+        *kept = *kept && awefd__adj_kept(b->m[s]);
+    }
+    return AWEFD_OK;
+}
+
 int awefd_batch_run_ckpt(awefd_batch *b, int ckpt)
 {
     if (!b) return awefd__fail(AWEFD_EINVAL, "NULL batch");
     HIPCHK(hipSetDevice(b->dev));
     int rc;
     if ((rc = shots_ready(b))) return rc;
-    int want = awefd__adj_interval(b->m, b->nshot, ckpt);
-    for (int s = 0; s < b->nshot; s++)
-        if ((rc = awefd__adj_ckpt_setup(b->m[s], want))) {
-            const int few = (int)ceil(sqrt((double)b->nt));
-            if (ckpt > 0 || want == few) return rc;
-            want = few;                      /* no memory for every field */
-            s = -1;
-        }
+    const int want = awefd__adj_interval(b->m, b->nshot, ckpt), few = (int)ceil(sqrt((double)b->nt));
+    int kept;
+    if ((rc = ckpt_setup(b, want, &kept))) return rc;
+    if (ckpt <= 0 && want == b->nt && !kept && few < want && (rc = ckpt_setup(b, few, &kept))) return rc;
+    for (int s = 0; s < b->nshot; s++) awefd__adj_keep(b->m[s], kept);
     const int K = awefd__adj_K(b->m[0]);
     if ((rc = batch_sync(b))) return rc;
-    if (K != b->K) {
+    if (K != b->K || kept != b->kept) {
         b->K = K;
+        b->kept = kept;
         b->nck = (b->nt + K - 1) / K;
         b->fwd_ok = b->bwd_ok = 0;
     }
@@ -1214,7 +1224,7 @@ int awefd_batch_run_ckpt(awefd_batch *b, int ckpt)
         return awefd__fail(AWEFD_ENOMEM, "batch checkpoint bases");
     for (int s = 0; s < b->nshot; s++)
         if (b->fwd_ck[s] != awefd__adj_ckpt(b->m[s], 0)) b->fwd_ok = 0;
-    if (K == b->nt) return run_kept(b);
+    if (kept) return run_kept(b);
     const int depth = ckpt_depth(b);
     if ((rc = capture_fwd(b, depth))) return rc;
     for (int s = 0; s < b->nshot; s++) b->fwd_ck[s] = awefd__adj_ckpt(b->m[s], 0);
@@ -1359,8 +1369,8 @@ static int capture_bwd(awefd_batch *b, int depth, int adepth)
     for (int g = 0; g < b->ngroup && !e; g++)
         for (int k = b->nck - 1; k >= 0 && !e; k--) {
             const int n0 = k * b->K, n1 = n0 + b->K < b->nt ? n0 + b->K : b->nt;
-            /* K = nt: the forward run kept the segment's fields */
-            int n = b->K < b->nt ? n0 : n1;
+            /* the forward run may have kept the one segment's fields */
+            int n = b->kept ? n1 : n0;
             for (; depth == 3 && n + 3 <= n1 - 1 && !e; n += 3)
                 e = awefd_launch_cart_batch_t3rc(b->d_shots, b->d_bshot2 + b->goff2[g], b->gnblk2[g], n, b->nop,
                                                  b->sse, b->rx, b->stream);
@@ -1401,7 +1411,7 @@ int awefd_batch_adjoint_grad(awefd_batch *b, const float *const *d_res, float *d
         awefd_model *m = b->m[s];
         if (!d_res[s]) return awefd__fail(AWEFD_EINVAL, "awefd_batch_adjoint_grad: residual %d is NULL", s);
         if ((rc = awefd__adj_ready(m, "awefd_batch_adjoint_grad"))) return rc;
-        if (awefd__adj_K(m) != b->K)
+        if (awefd__adj_K(m) != b->K || (b->kept && !awefd__adj_kept(m)))
             return awefd__fail(AWEFD_ESTATE, "awefd_batch_adjoint_grad: shot %d was not run by awefd_batch_run_ckpt", s);
         if (m->p.n[0] != m0->p.n[0] || m->p.n[1] != m0->p.n[1] || m->nb != m0->nb || m->ld != m0->ld)
             return awefd__fail(AWEFD_EINVAL, "awefd_batch_adjoint_grad: shot %d has another grid (the gradient "

@@ -160,6 +160,8 @@ int  awefd__polar_run(awefd_model *m, float *dtr, int *done);
 void   awefd__adjoint_free(awefd_model *m);
 int    awefd__adj_ckpt_setup(awefd_model *m, int ckpt);
 int    awefd__adj_interval(awefd_model *const *ms, int n, int ckpt);
+int    awefd__adj_kept(const awefd_model *m);
+void   awefd__adj_keep(awefd_model *m, int kept);
 int    awefd__adj_kept_end(awefd_model *m, hipStream_t stream);
 int    awefd__adj_kept_traces(awefd_model *m, float *dtr, hipStream_t stream);
 float *awefd__adj_ckpt(const awefd_model *m, int k);
