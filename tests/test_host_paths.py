@@ -163,3 +163,16 @@ def test_a_batch_that_keeps_every_step_of_some_shots_only(stub):
     b.close()
     for m in ms:
         m.close()
+
+
+def test_traces_of_more_steps_than_a_grid_has_rows(stub, monkeypatch):
+    """The trace rows of a run that kept its fields are rows of a launch's
+    grid, of which there are at most 65,535."""
+    monkeypatch.setenv("AWEFD_RESIDENT", "0")
+    nt = 140000
+    with _model(nt=nt, n=(5, 5), nb=1, fdorder=2, nr=1) as m:
+        tr, tp = _dev(nt, 1)
+        L.check(m.lib.awefd_run_ckpt(m.h, tp, nt))
+        assert stub.get("rows") == nt
+        assert stub.get("max_rows") <= 65535
+        np.testing.assert_array_equal(tr[:, 0], np.arange(nt, dtype=np.float32))     # row n of field n

@@ -275,14 +275,21 @@ int awefd__adj_kept_end(awefd_model *m, hipStream_t stream)
     return AWEFD_OK;
 }
 
-/* Traces of a run that kept fields 0 .. nt-1. */
+/* Traces of a run that kept fields 0 .. nt-1, as many rows a launch as a grid
+ * has in y. */
 int awefd__adj_kept_traces(awefd_model *m, float *dtr, hipStream_t stream)
 {
     const adj_state *s = state(m);
+    const int nt = m->p.nt, most = 65535;
     awefd_cart_args a;
     awefd__cart_args(m, &a);
-    const int e = awefd_launch_cart_traces(&a, s->ck, s->seg, m->nalloc, m->p.nt, dtr, stream);
-    return e ? awefd__fail(AWEFD_EHIP, "traces: %s", hipGetErrorString((hipError_t)e)) : AWEFD_OK;
+    for (int n = 0; n < nt; n += min_i(most, nt - n)) {
+        const float *next = n + 1 < nt ? kept_field(s, m->nalloc, n + 1) : NULL;
+        const int e = awefd_launch_cart_traces(&a, kept_field(s, m->nalloc, n), next, m->nalloc, min_i(most, nt - n),
+                                               dtr + (size_t)n * a.nr, stream);
+        if (e) return awefd__fail(AWEFD_EHIP, "traces: %s", hipGetErrorString((hipError_t)e));
+    }
+    return AWEFD_OK;
 }
 
 /* Forward run that keeps every field: the resident loop where the model takes
