@@ -22,7 +22,7 @@ static hipError_t last;
 
 void stub_reset(long fail_at, size_t fail_above)
 {
-    stub_allocs = stub_bytes = stub_resident = stub_adjoint = stub_steps = stub_rows = stub_max_rows = stub_recomputed = 0;
+    stub_allocs = stub_resident = stub_adjoint = stub_steps = stub_rows = stub_max_rows = stub_recomputed = 0;
     stub_fail_at = fail_at;
     stub_fail_above = fail_above;
     stub_launch_error = stub_give_up = 0;
@@ -33,8 +33,10 @@ static hipError_t take(void **p, size_t n)
 {
     stub_allocs++;
     if (stub_allocs == stub_fail_at || (stub_fail_above && n > stub_fail_above)) return last = hipErrorOutOfMemory;
-    *p = calloc(1, n > 0 ? n : 1);
-    if (!*p) return last = hipErrorOutOfMemory;
+    char *b = calloc(1, n + 64);
+    if (!b) return last = hipErrorOutOfMemory;
+    memcpy(b, &n, sizeof n);                           /* its size ahead of it */
+    *p = b + 64;
     stub_bytes += (long)n;
     return hipSuccess;
 }
@@ -48,8 +50,16 @@ hipError_t hipGetLastError(void)
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : e ? "other error" : "no error"; }
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return take(p, n); }
-hipError_t hipFree(void *p) { free(p); return hipSuccess; }
-hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipFree(void *p)
+{
+    size_t n;
+    if (!p) return hipSuccess;
+    memcpy(&n, (char *)p - 64, sizeof n);
+    stub_bytes -= (long)n;
+    free((char *)p - 64);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st) { (void)st; return hipMemcpy(d, s, n, k); }
 hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind k)

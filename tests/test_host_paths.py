@@ -176,3 +176,91 @@ def test_traces_of_more_steps_than_a_grid_has_rows(stub, monkeypatch):
         assert stub.get("rows") == nt
         assert stub.get("max_rows") <= 65535
         np.testing.assert_array_equal(tr[:, 0], np.arange(nt, dtype=np.float32))     # row n of field n
+
+
+def _passes(kind, stub, fail_at):
+    """Set-up, two runs and (cart2d) a gradient with allocation `fail_at`
+    refused; whether every call went through, and the allocations asked for."""
+    stub.reset(fail_at=fail_at)
+    try:
+        with _model(kind=kind) as m:
+            m.run()
+            m.run()
+            if kind == "cart2d":
+                _grad(m, 9)
+                _grad(m, 9)
+    except L.AwefdError as e:
+        assert "out of memory" in str(e)
+        return False, stub.get("allocs")
+    return True, stub.get("allocs")
+
+
+@pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
+def test_the_resident_loops_memory_is_optional(kind, stub, monkeypatch):
+    """Calls fail for the allocations that the loop of one launch per step
+    needs too, and for no others."""
+    failed, asked = {}, {}
+    for on in ("0", "1"):
+        monkeypatch.setenv("AWEFD_RESIDENT", on)
+        ok, asked[on] = _passes(kind, stub, 0)
+        assert ok and (stub.get("resident") > 0) == (on == "1")
+        failed[on] = sum(not _passes(kind, stub, n)[0] for n in range(1, asked[on] + 1))
+    assert asked["1"] > asked["0"]
+    assert failed["1"] == failed["0"] > 0
+    if kind == "spher2d":
+        assert failed["0"] == asked["0"] - 1         # the receivers near the sources: separate launches then
+
+
+@pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
+def test_a_model_without_the_resident_loops_memory(kind, stub):
+    """Whichever allocation was refused: a run without it takes the other
+    loop; with memory again (polar: and its setters called again) the resident
+    one."""
+    asked, lacked = _passes(kind, stub, 0)[1], 0
+    for n in range(1, asked + 1):
+        stub.reset(fail_at=n)
+        try:
+            m = _model(kind=kind)
+        except L.AwefdError:
+            continue
+        stub.reset()
+        m.traces_dev()
+        stub.reset(fail_above=1)
+        m.run()
+        lacked += stub.get("resident") == 0
+        stub.reset()
+        if kind == "spher2d":
+            m.set_model(np.full((40, 30), 1.7e8, np.float32))
+            x = np.array([[3387.5e3, 0.785]], np.float32)
+            m.set_sources(x)
+            m.set_receivers(x)
+        m.run()
+        assert stub.get("resident") == 1
+        m.close()
+    assert lacked > 0
+
+
+def test_shots_of_a_batch_hold_no_rims(stub, monkeypatch):
+    held = []
+    for on in ("0", "1"):
+        monkeypatch.setenv("AWEFD_RESIDENT", on)
+        before = stub.get("bytes")
+        ms = [_model(nt=30) for _ in range(2)]
+        b = awefd.Batch(ms)
+        for m in ms:
+            m.set_sources(np.array([[20.0, 20.0]], np.float32))
+        res, rp = _dev(30, 5)
+        g, gp = _dev(40, 30)
+        b.run()
+        b.run_ckpt(0)
+        b.adjoint_grad([rp, rp], gp)
+        held.append(stub.get("bytes") - before)
+        ms[0].run()                                  # one of them alone
+        _grad(ms[0], 30)
+        assert stub.get("resident") == (2 if on == "1" else 0) and stub.get("adjoint") == (on == "1")
+        b.close()
+        for m in ms:
+            m.close()
+        assert stub.get("bytes") == before
+        stub.reset()
+    assert 0 <= held[1] - held[0] < 2 * 4096         # two shots' flags and point tables

@@ -395,26 +395,42 @@ static void adj2_tiles(const awefd_model *m, int *ntz2, int *ntx2)
     *ntx2 = (m->np[1] + sx - 1) / sx;
 }
 
-/* The tile of the resident adjoint loop, and its rim words: for the models
- * whose forward loop is resident, the fewest rows per wave whose blocks fit
- * one per CU.  rt.on = 0: the loop of one launch per step. */
-static void resadj_pick(awefd_model *m, adj_state *s)
+/* The resident adjoint loop's tile, rim words and point lists, for the models
+ * whose forward loop is resident: the fewest rows per wave whose blocks fit
+ * one per CU.  rt.on = 0: the loop of one launch per step, also where there is
+ * no memory.  (Not for a batch, whose backward pass never runs it.) */
+static void resadj_prepare(awefd_model *m, adj_state *s)
 {
     static const int list[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 0};
+    awefd_res_tile *t = &s->rt;
     int cus = 0;
-    if (s->E.p) return;                        /* the grid's: picked before */
-    s->rt.on = 0;
-    if (!m->res.on || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev) != hipSuccess) return;
-    for (const int *rx = list; *rx; rx++) {
-        awefd__res_tile_of(m, m->nop, *rx, 1, AWEFD_RES_NWAVE, &s->rt);
-        if (s->rt.on && (long)s->rt.ntz * s->rt.ntx <= cus) break;
-        s->rt.on = 0;
+    if (s->rinjr) return;                      /* the lists of these points */
+    if (!s->E.p) {
+        t->on = 0;
+        if (!m->res.on || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->dev) != hipSuccess)
+            return;
+        for (const int *rx = list; *rx; rx++) {
+            awefd__res_tile_of(m, m->nop, *rx, 1, AWEFD_RES_NWAVE, t);
+            if (t->on && (long)t->ntz * t->ntx <= cus) break;
+            t->on = 0;
+        }
+        if (!t->on) return;
+        const size_t bytes = sizeof(unsigned long long) * 2 * (size_t)t->words * t->ntz * t->ntx;
+        s->tag = 1;
+        t->on = awefd__resadj_blocks(m->nop, t->rx) >= 1 && !awefd__res_grow(&s->E, bytes) &&
+                !awefd_launch_fill(s->E.p, (long)(bytes / sizeof(float)), 0.f, m->stream);
     }
-    if (!s->rt.on) return;
-    const size_t bytes = sizeof(unsigned long long) * 2 * (size_t)s->rt.words * s->rt.ntz * s->rt.ntx;
-    s->tag = 1;
-    s->rt.on = awefd__resadj_blocks(m->nop, s->rt.rx) >= 1 && !awefd__res_grow(&s->E, bytes) &&
-               !awefd_launch_fill(s->E.p, (long)(bytes / sizeof(float)), 0.f, m->stream);
+    if (!t->on) return;
+    const int nw = t->ntx * t->nw;
+    if (!point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, t->ntz, nw, t->zw, t->rx, 0, &s->rinjr, &s->rbegr) &&
+        !point_buckets(m, m->ns, m->h_sj, m->h_sw, m->p.expl, t->ntz, nw, t->zw, t->rx, 0, &s->sinjr, &s->sbegr))
+        return;
+    hipFree(s->rinjr); hipFree(s->sinjr); hipFree(s->rbegr); hipFree(s->sbegr);
+    s->rinjr = s->sinjr = NULL;
+    s->rbegr = s->sbegr = NULL;
+    hipFree(s->E.p);                           /* no memory: picked again next time */
+    memset(&s->E, 0, sizeof s->E);
+    t->on = 0;
 }
 
 /* Every backward step of a run that kept its fields, as one launch; *done = 0:
@@ -424,7 +440,8 @@ static int resadj_run(awefd_model *m, adj_state *s, const awefd_adj2d_args *g, i
     awefd_resadj_args a;
     int rc;
     *done = 0;
-    if (!s->rt.on || !m->res.on) return AWEFD_OK;
+    resadj_prepare(m, s);
+    if (!s->rt.on || !m->res.on || awefd__res_flag(m)) return AWEFD_OK;
     memset(&a, 0, sizeof a);
     a.nz = g->nz;
     a.nx = g->nx;
@@ -509,15 +526,6 @@ int awefd__adj_prepare(awefd_model *m)
         if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, ntz2, ntx2, 64, AWEFD_ADJ2_ROWS, m->nop, &s->sinj2,
                                 &s->sbeg2)))
             return rc;
-        resadj_pick(m, s);
-        if (s->rt.on) {
-            const awefd_res_tile *t = &s->rt;
-            const int nw = t->ntx * t->nw;
-            if ((rc = point_buckets(m, m->nr, m->h_rj, m->h_rw, 0, t->ntz, nw, t->zw, t->rx, 0, &s->rinjr, &s->rbegr)))
-                return rc;
-            if ((rc = point_buckets(m, m->ns, m->h_sj, m->h_sw, ex, t->ntz, nw, t->zw, t->rx, 0, &s->sinjr, &s->sbegr)))
-                return rc;
-        }
         s->lists_ok = 1;
         s->lists_gen = m->bgen;
     }

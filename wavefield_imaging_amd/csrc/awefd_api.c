@@ -631,6 +631,9 @@ static int set_points(awefd_model *m, int which, int n, const float *coords)
         free(m->h_rsinc);
         m->h_rsinc = sp;
     }
+    /* the resident loop's tables are now stale */
+    if (which == 0 || m->inj_rec) m->res.src_ok = 0;
+    if (which == 1) m->res.rec_ok = 0;
     if (which == 0) {
         free(m->h_sj); free(m->h_sw);
         m->h_sj = j; m->h_sw = w; m->ns = n;
@@ -719,7 +722,7 @@ static int cart_build_inj(awefd_model *m)
     if (!rc) rc = upload(m, (void **)&m->d_ibeg, ibeg, sizeof(int) * (nbucket + 1));
     m->ninj = n;
     free(e); free(ibeg);
-    return rc ? rc : awefd__res_set_sources(m);
+    return rc;
 }
 
 int awefd_set_sources(awefd_model *m, int ns, const float *coords)
@@ -729,6 +732,7 @@ int awefd_set_sources(awefd_model *m, int ns, const float *coords)
     HIPCHK(hipSetDevice(m->dev));
     if (!is_cart(m)) rc = awefd__spher_set_sources(m);
     else if (!m->inj_rec) rc = cart_build_inj(m);
+    if (!rc && is_cart(m)) awefd__res_prepare(m);
     if (!rc) m->src_set = 1;
     const int rd = setter_done(m);
     return rc ? rc : rd;
@@ -744,7 +748,8 @@ int awefd_set_receivers(awefd_model *m, int nr, const float *coords)
     if (!rc && m->sinc)
         rc = upload(m, (void **)&m->d_rsinc, m->h_rsinc, sizeof(awefd_sinc_pt) * (nr > 0 ? nr : 1));
     if (!rc && m->inj_rec) rc = cart_build_inj(m);
-    if (!rc) rc = is_cart(m) ? awefd__res_set_receivers(m) : awefd__spher_set_receivers(m);
+    if (!rc && is_cart(m)) awefd__res_prepare(m);
+    else if (!rc) rc = awefd__spher_set_receivers(m);
     if (!rc) m->rec_set = 1;
     const int rd = setter_done(m);
     return rc ? rc : rd;

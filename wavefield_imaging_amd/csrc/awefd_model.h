@@ -14,9 +14,12 @@ typedef struct {
     size_t cap;
 } awefd_res_buf;
 
-/* resident 2-D loop (awefd_resident.c): its tile, rim words, point tables */
+/* resident 2-D loop (awefd_resident.c): its tile, rim words, point tables.
+ * Its memory is optional: a run without it takes the loop of one launch per
+ * step. */
 typedef struct {
-    int on;
+    int on;                       /* the grid has a tile                     */
+    int src_ok, rec_ok, one_ok;   /* the tables are those of the last setter */
     awefd_res_tile t;
     awefd_res_buf E, src, rec, one;   /* one: polar one-way nodes            */
     size_t inj_off, idx_off, one_off;
@@ -140,8 +143,6 @@ int  awefd__res_launch(int nop, const awefd_res_tile *t, const awefd_res_args *a
 int  awefd__res_blocks(int nop, const awefd_res_tile *t, int vd);
 int  awefd__res_create(awefd_model *m);
 void awefd__res_free(awefd_model *m);
-int  awefd__res_set_sources(awefd_model *m);
-int  awefd__res_set_receivers(awefd_model *m);
 int  awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *out, size_t *inj_off);
 int  awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *out, size_t *idx_off);
 int  awefd__res_tags(awefd_res_buf *E, unsigned *tag, int nt, hipStream_t s, unsigned *tag0);
@@ -151,6 +152,8 @@ int  awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done);
 int  awefd__res_grow(awefd_res_buf *b, size_t bytes);
 void awefd__res_tile_of(const awefd_model *m, int nop, int rx, int S, int nw, awefd_res_tile *t);
 int  awefd__res_buffers(awefd_model *m);
+int  awefd__res_flag(awefd_model *m);
+void awefd__res_prepare(awefd_model *m);
 void awefd__res_wait(unsigned *wmask, long long *wticks);
 int  awefd__res_finish(awefd_model *m, int launched, int *done);
 /* resident polar loop (spher_host.c) */

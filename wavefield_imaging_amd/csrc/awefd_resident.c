@@ -102,18 +102,37 @@ int awefd__res_blocks(int nop, const awefd_res_tile *t, int vd)
     return BLOCKS[nop - 1](t->rx, t->S, vd);
 }
 
-/* rim words and the stop flag of the tile picked; on */
+/* The flag a block raises when it gives up waiting. */
+int awefd__res_flag(awefd_model *m)
+{
+    awefd_res *r = &m->res;
+    if (r->stop) return AWEFD_OK;
+    const hipError_t e = hipHostMalloc((void **)&r->stop, sizeof(unsigned), hipHostMallocDefault);
+    if (e != hipSuccess) {
+        r->stop = NULL;
+        return awefd__fail(AWEFD_ENOMEM, "resident loop's flag: %s", hipGetErrorString(e));
+    }
+    *r->stop = 0;
+    return AWEFD_OK;
+}
+
+/* Rim words and the flag of the tile picked.  The words are taken by the first
+ * run: a shot that only ever runs in a batch needs none (2.6 MB beside 5.6 MB of
+ * fields for 500 x 900 nodes; 60 uneven shots held 835 MB instead of 596). */
 int awefd__res_buffers(awefd_model *m)
 {
     awefd_res *r = &m->res;
+    int rc = awefd__res_flag(m);
+    if (rc || r->E.p) return rc;
     const size_t eb = sizeof(unsigned long long) * 2 * (size_t)r->t.words * r->t.ntz * r->t.ntx;
-    if (awefd__res_grow(&r->E, eb)) return AWEFD_ENOMEM;
+    if ((rc = awefd__res_grow(&r->E, eb))) return rc;
     const int e = awefd_launch_fill(r->E.p, (long)(eb / sizeof(float)), 0.f, m->stream);
-    if (e) return awefd__fail(AWEFD_EHIP, "resident rims: %s", hipGetErrorString((hipError_t)e));
-    HIPCHK(hipHostMalloc((void **)&r->stop, sizeof(unsigned), hipHostMallocDefault));
-    *r->stop = 0;
+    if (e) {
+        hipFree(r->E.p);
+        memset(&r->E, 0, sizeof r->E);
+        return awefd__fail(AWEFD_EHIP, "resident rims: %s", hipGetErrorString((hipError_t)e));
+    }
     r->tag = 1;
-    r->on = 1;
     if (getenv("AWEFD_VERBOSE"))
         fprintf(stderr, "awefd: resident 2-D loop: %d x %d blocks of %d waves, %d rows per wave, %d steps per exchange\n",
                 r->t.ntz, r->t.ntx, r->t.nw, r->t.rx, r->t.S);
@@ -132,8 +151,9 @@ int awefd__res_create(awefd_model *m)
     const int vd = !m->p.cden;
     awefd__res_pick(m, vd, cus, &r->t);
     if (!r->t.on && vd) awefd__res_pick(m, 0, cus, &r->t);
-    if (!r->t.on || awefd__res_blocks(m->nop, &r->t, 0) < 1) return AWEFD_OK;
-    return awefd__res_buffers(m);
+    r->on = r->t.on && awefd__res_blocks(m->nop, &r->t, 0) >= 1;
+    awefd__res_prepare(m);
+    return AWEFD_OK;
 }
 
 void awefd__res_free(awefd_model *m)
@@ -223,16 +243,27 @@ int awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf 
     return rc;
 }
 
-int awefd__res_set_sources(awefd_model *m)
+/* The tables that a setter made stale and whose points are set. */
+static int tables(awefd_model *m)
 {
     awefd_res *r = &m->res;
-    return r->on ? awefd__res_sources(m, &r->t, &r->src, &r->inj_off) : AWEFD_OK;
+    int rc = AWEFD_OK;
+    if (!r->src_ok && (m->inj_rec ? m->h_rj : m->h_sj)) {
+        rc = awefd__res_sources(m, &r->t, &r->src, &r->inj_off);
+        r->src_ok = !rc;
+    }
+    if (!rc && !r->rec_ok && m->h_rj) {
+        rc = awefd__res_receivers(m, &r->t, &r->rec, &r->idx_off);
+        r->rec_ok = !rc;
+    }
+    return rc;
 }
 
-int awefd__res_set_receivers(awefd_model *m)
+/* Ahead of a run, by awefd_create and the point setters: the flag and the
+ * tables; what fails is left to the run, which does without. */
+void awefd__res_prepare(awefd_model *m)
 {
-    awefd_res *r = &m->res;
-    return r->on ? awefd__res_receivers(m, &r->t, &r->rec, &r->idx_off) : AWEFD_OK;
+    if (m->res.on && !awefd__res_flag(m)) (void)tables(m);
 }
 
 /* First tag of a run of nt steps over the rims of E: tags only grow, so the
@@ -326,7 +357,7 @@ int awefd__res_run(awefd_model *m, float *dtr, float *fields, int *done)
     awefd_res *r = &m->res;
     awefd_res_args a;
     *done = 0;
-    if (!r->on) return AWEFD_OK;
+    if (!r->on || awefd__res_buffers(m) || tables(m)) return AWEFD_OK;
     awefd__res_args(m, &r->t, &r->src, r->inj_off, &r->rec, r->idx_off, dtr, &a);
     a.F = fields;
     a.nal = m->nalloc;

@@ -53,7 +53,7 @@ typedef struct {
 
 static spher_state *st(awefd_model *m) { return (spher_state *)m->spher; }
 static int build_injection(awefd_model *m);
-static int build_conflicts(awefd_model *m);
+static void build_conflicts(awefd_model *m);
 static int polar_create(awefd_model *m);
 static int polar_sources(awefd_model *m, const long *node, int n);
 static int polar_receivers(awefd_model *m);
@@ -329,7 +329,7 @@ int awefd__spher_set_model(awefd_model *m, const float *vel)
                 t[5][(long)ith * n1 + ir] = awefd_oneway_spher(vp[(long)(n2 - NOP - 1) * Y + ith * Z + ir], dt, dph);
             }
     }
-    if (!rc) rc = polar_oneway(m, t);
+    m->res.one_ok = !rc && !polar_oneway(m, t);
     for (int i = 0; i < 6; i++) {
         if (!rc) rc = up(&s->d_ow[i], t[i], sizeof(float) * sz[i]);
         free(t[i]);
@@ -364,14 +364,16 @@ int awefd__spher_set_receivers(awefd_model *m)
     }
     int rc = up(&s->d_rrtp, h, sizeof(int) * 3 * (m->nr > 0 ? m->nr : 1));
     free(h);
-    if (!rc) rc = polar_receivers(m);
-    return rc ? rc : s->inj_dirty || !m->h_sj ? AWEFD_OK : build_conflicts(m);
+    m->res.rec_ok = !rc && !polar_receivers(m);
+    if (!rc && !s->inj_dirty && m->h_sj) build_conflicts(m);
+    return rc;
 }
 
 /* The box of the injection nodes and the receivers that read a node of it
  * (the extraction has to read them before the next injection); built by
- * whichever of the point setters comes last. */
-static int build_conflicts(awefd_model *m)
+ * whichever of the point setters comes last.  Without memory for the list:
+ * more of them than the fused launch takes. */
+static void build_conflicts(awefd_model *m)
 {
     spher_state *s = st(m);
     const int ax[3] = {1, 0, 2};                   /* (r, theta, phi) of the point map */
@@ -384,20 +386,19 @@ static int build_conflicts(awefd_model *m)
             if (j + 1 > s->box[2 * k + 1]) s->box[2 * k + 1] = j + 1;
         }
     }
-    s->nconf = 0;
-    int *h = malloc(sizeof(int) * (m->nr > 0 ? m->nr : 1));
-    if (!h) return awefd__fail(AWEFD_ENOMEM, "receivers near sources");
+    s->nconf = AWEFD_SPHER_FUSE_CONF + 1;
+    int n = 0, *h = malloc(sizeof(int) * (m->nr > 0 ? m->nr : 1));
+    if (!h) return;
     for (int r = 0; r < m->nr; r++) {
         int hit = 1;
         for (int k = 0; k < m->ndim; k++) {
             const int j = m->h_rj[3 * r + ax[k]];
             hit = hit && j + 1 >= s->box[2 * k] && j <= s->box[2 * k + 1];
         }
-        if (hit) h[s->nconf++] = r;
+        if (hit) h[n++] = r;
     }
-    const int rc = up(&s->d_conf, h, sizeof(int) * s->nconf);
+    if (!up(&s->d_conf, h, sizeof(int) * n)) s->nconf = n;
     free(h);
-    return rc;
 }
 
 /* Reflectivity |v0 - vk| / (v0 + vk) of the first neighbour k whose velocity
@@ -497,11 +498,12 @@ static int build_injection(awefd_model *m)
         rc = up(&s->d_inode, node, sizeof(long) * (nn > 0 ? nn : 1));
         if (!rc) rc = up(&s->d_ibeg, ibeg, sizeof(int) * (nn + 1));
         if (!rc) rc = up(&s->d_iw, iw, sizeof(float) * 2 * (n > 0 ? n : 1));
-        if (!rc) rc = polar_sources(m, node, nn);
+        m->res.src_ok = !rc && !polar_sources(m, node, nn);
     }
     free(e); free(node); free(ibeg); free(iw);
     if (!rc) s->inj_dirty = 0;
-    return rc || !m->h_rj ? rc : build_conflicts(m);
+    if (!rc && m->h_rj) build_conflicts(m);
+    return rc;
 }
 
 static void spher_args(const awefd_model *m, awefd_spher_args *a)
@@ -677,7 +679,9 @@ static int polar_create(awefd_model *m)
                 continue;
             free(polar_items(m, t, NULL, &off, &bytes, &fits));
             if (!fits || awefd__polar_blocks(*rx, S) < 1) continue;
-            return awefd__res_buffers(m);
+            r->on = 1;
+            (void)awefd__res_flag(m);
+            return AWEFD_OK;
         }
     }
     return AWEFD_OK;
@@ -778,6 +782,7 @@ int awefd__polar_run(awefd_model *m, float *dtr, int *done)
     *done = 0;
     if (s->inj_dirty && (rc = build_injection(m))) return rc;
     if (!s->d_rrtp) return awefd__fail(AWEFD_ESTATE, "receivers not set");
+    if (!r->one_ok || !r->src_ok || !r->rec_ok || awefd__res_buffers(m)) return AWEFD_OK;
     memset(&a, 0, sizeof a);
     a.n1 = m->np[0];
     a.n2 = m->np[1];
