@@ -264,3 +264,35 @@ def test_shots_of_a_batch_hold_no_rims(stub, monkeypatch):
         assert stub.get("bytes") == before
         stub.reset()
     assert 0 <= held[1] - held[0] < 2 * 4096         # two shots' flags and point tables
+
+
+@pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
+def test_launch_errors_of_a_resident_loop(kind, stub):
+    """A device that cannot hold the blocks (720) or launch them together
+    (801): the other loop, from then on.  Any other error is the run's."""
+    for code in (720, 801):
+        with _model(kind=kind) as m:
+            stub.reset()
+            stub.set("launch_error", code)
+            m.run()
+            m.run()
+            assert stub.get("resident") == 1
+    with _model(kind=kind) as m:
+        stub.reset()
+        stub.set("launch_error", 719)                # an earlier kernel failed
+        with pytest.raises(L.AwefdError, match="resident"):
+            m.run()
+
+
+def test_launch_errors_of_the_resident_adjoint(stub):
+    with _model() as m:
+        L.check(m.lib.awefd_run_ckpt(m.h, None, 9))
+        res, rp = _dev(m.nt, m.nr)
+        g, gp = _dev(40, 30)
+        stub.set("launch_error", 719)
+        assert m.lib.awefd_adjoint_grad(m.h, rp, gp) == -2
+        assert b"resident adjoint" in m.lib.awefd_last_error()
+        stub.set("launch_error", 720)
+        for _ in range(2):
+            L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
+        assert stub.get("adjoint") == 2

@@ -473,8 +473,11 @@ static int resadj_run(awefd_model *m, adj_state *s, const awefd_adj2d_args *g, i
     a.stop = m->res.stop;
     awefd__res_wait(&a.wmask, &a.wticks);
     if ((rc = awefd__res_tags(&s->E, &s->tag, a.nt, m->stream, &a.tag0))) return rc;
-    if (awefd__resadj_launch(&a, a.ntz * a.ntx, m->nop, s->rt.rx, m->stream)) {
-        (void)hipGetLastError();               /* this device cannot hold the blocks */
+    const int l = awefd__resadj_launch(&a, a.ntz * a.ntx, m->nop, s->rt.rx, m->stream);
+    if (l) {
+        (void)hipGetLastError();
+        if (!awefd__res_refused(l))
+            return awefd__fail(AWEFD_EHIP, "resident adjoint: %s", hipGetErrorString((hipError_t)l));
         s->rt.on = 0;
         return AWEFD_OK;
     }

@@ -329,13 +329,22 @@ void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_
     awefd__res_wait(&a->wmask, &a->wticks);
 }
 
+/* Whether a cooperative launch was refused for what the device can hold or do
+ * (the caller then has another loop), not for an error of its own. */
+int awefd__res_refused(int e)
+{
+    return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported || e == hipErrorInvalidConfiguration ||
+           e == hipErrorInvalidValue || e == hipErrorLaunchOutOfResources || e == hipErrorOutOfMemory;
+}
+
 /* After a launch: its wait, and whether every block went through (*done). */
 int awefd__res_finish(awefd_model *m, int launched, int *done)
 {
     awefd_res *r = &m->res;
     if (launched) {
-        /* not launched: this device cannot hold the blocks */
         (void)hipGetLastError();
+        if (!awefd__res_refused(launched))
+            return awefd__fail(AWEFD_EHIP, "resident loop: %s", hipGetErrorString((hipError_t)launched));
         r->on = 0;
         return AWEFD_OK;
     }
