@@ -296,3 +296,36 @@ def test_launch_errors_of_the_resident_adjoint(stub):
         for _ in range(2):
             L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
         assert stub.get("adjoint") == 2
+
+
+@pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
+def test_a_loop_that_gave_up_is_not_tried_again(kind, stub, monkeypatch, capfd):
+    """A wait that ends takes 4 s; a handle whose blocks did not get on pays
+    it once, and says so."""
+    monkeypatch.setenv("AWEFD_VERBOSE", "1")
+    with _model(kind=kind) as m:
+        stub.reset()
+        stub.set("give_up", 1)
+        m.run()
+        assert stub.get("resident") == 1
+        m.run()
+        assert stub.get("resident") == 1
+    assert "resident loop off" in capfd.readouterr().err
+
+
+def test_an_adjoint_that_gave_up_is_not_tried_again(stub, monkeypatch, capfd):
+    monkeypatch.setenv("AWEFD_VERBOSE", "1")
+    with _model() as m:
+        stub.reset()
+        _grad(m, 9)
+        assert stub.get("resident") == 1 and stub.get("adjoint") == 1
+        stub.set("give_up", 1)
+        res, rp = _dev(m.nt, m.nr)
+        g, gp = _dev(40, 30)
+        for _ in range(2):
+            L.check(m.lib.awefd_adjoint_grad(m.h, rp, gp))
+        assert stub.get("adjoint") == 2
+        stub.set("give_up", 0)
+        _grad(m, 9)                                  # the forward loop did get on
+        assert stub.get("resident") == 2 and stub.get("adjoint") == 2
+    assert "resident adjoint off" in capfd.readouterr().err

@@ -18,6 +18,7 @@
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
 #include <math.h>
+#include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -419,6 +420,9 @@ static void resadj_prepare(awefd_model *m, adj_state *s)
         s->tag = 1;
         t->on = awefd__resadj_blocks(m->nop, t->rx) >= 1 && !awefd__res_grow(&s->E, bytes) &&
                 !awefd_launch_fill(s->E.p, (long)(bytes / sizeof(float)), 0.f, m->stream);
+        if (t->on && getenv("AWEFD_VERBOSE"))
+            fprintf(stderr, "awefd: resident adjoint: %d x %d blocks of %d waves, %d rows per wave\n", t->ntz, t->ntx,
+                    t->nw, t->rx);
     }
     if (!t->on) return;
     const int nw = t->ntx * t->nw;
@@ -478,13 +482,14 @@ static int resadj_run(awefd_model *m, adj_state *s, const awefd_adj2d_args *g, i
         (void)hipGetLastError();
         if (!awefd__res_refused(l))
             return awefd__fail(AWEFD_EHIP, "resident adjoint: %s", hipGetErrorString((hipError_t)l));
-        s->rt.on = 0;
+        awefd__res_off(&s->rt.on, "adjoint", hipGetErrorString((hipError_t)l));
         return AWEFD_OK;
     }
     const hipError_t e = hipStreamSynchronize(m->stream);
     if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "resident adjoint: %s", hipGetErrorString(e));
     *done = *(volatile unsigned *)m->res.stop == 0;
     *m->res.stop = 0;
+    if (!*done) awefd__res_off(&s->rt.on, "adjoint", "a block gave up waiting");
     return AWEFD_OK;
 }
 

@@ -337,7 +337,15 @@ int awefd__res_refused(int e)
            e == hipErrorInvalidValue || e == hipErrorLaunchOutOfResources || e == hipErrorOutOfMemory;
 }
 
-/* After a launch: its wait, and whether every block went through (*done). */
+/* The resident loop `who` is not tried again by this handle: *on = 0. */
+void awefd__res_off(int *on, const char *who, const char *why)
+{
+    *on = 0;
+    if (getenv("AWEFD_VERBOSE")) fprintf(stderr, "awefd: resident %s off: %s\n", who, why);
+}
+
+/* After a launch: its wait, and whether every block went through (*done).  A
+ * block that gave up waited for 4 s, so that is not tried twice. */
 int awefd__res_finish(awefd_model *m, int launched, int *done)
 {
     awefd_res *r = &m->res;
@@ -345,12 +353,13 @@ int awefd__res_finish(awefd_model *m, int launched, int *done)
         (void)hipGetLastError();
         if (!awefd__res_refused(launched))
             return awefd__fail(AWEFD_EHIP, "resident loop: %s", hipGetErrorString((hipError_t)launched));
-        r->on = 0;
+        awefd__res_off(&r->on, "loop", hipGetErrorString((hipError_t)launched));
         return AWEFD_OK;
     }
     HIPCHK(hipStreamSynchronize(m->stream));
     if (*(volatile unsigned *)r->stop) {
         *r->stop = 0;
+        awefd__res_off(&r->on, "loop", "a block gave up waiting");
         return AWEFD_OK;
     }
     m->steps_done = m->nsteps;
