@@ -2,9 +2,10 @@
  * A HIP runtime and kernel launchers without a GPU, for the host code's own
  * paths (test_host_paths.py): device memory is host memory, launches count
  * themselves and do nothing.  Allocation `fail_at` (counted from 1, by
- * stub_reset) and any of more than `fail_above` bytes are refused; as in HIP,
- * the error of a failed call stays the thread's last error until
- * hipGetLastError takes it, and a launcher reports it.
+ * stub_reset) and any of more than `fail_above` bytes are refused, and
+ * the synchronous copies while another thread captures (stub_capturing), as HIP
+ * refuses them; as in HIP too, the error of a failed call stays the thread's
+ * last error until hipGetLastError takes it, and a launcher reports it.
  */
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
@@ -17,7 +18,7 @@
 
 long stub_allocs, stub_fail_at, stub_bytes, stub_resident, stub_adjoint, stub_steps, stub_rows, stub_max_rows, stub_recomputed;
 size_t stub_fail_above;
-int stub_launch_error, stub_give_up;
+int stub_launch_error, stub_give_up, stub_capturing;
 static hipError_t last;
 
 void stub_reset(long fail_at, size_t fail_above)
@@ -25,7 +26,7 @@ void stub_reset(long fail_at, size_t fail_above)
     stub_allocs = stub_resident = stub_adjoint = stub_steps = stub_rows = stub_max_rows = stub_recomputed = 0;
     stub_fail_at = fail_at;
     stub_fail_above = fail_above;
-    stub_launch_error = stub_give_up = 0;
+    stub_launch_error = stub_give_up = stub_capturing = 0;
     last = hipSuccess;
 }
 
@@ -60,13 +61,21 @@ hipError_t hipFree(void *p)
     return hipSuccess;
 }
 hipError_t hipHostFree(void *p) { return hipFree(p); }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st) { (void)st; return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
+{
+    (void)k; (void)st;
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k)
+{
+    return stub_capturing ? (last = hipErrorStreamCaptureImplicit) : hipMemcpyAsync(d, s, n, k, NULL);
+}
 hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind k)
 {
-    (void)k;
-    for (size_t i = 0; i < h; i++) memcpy((char *)d + i * dp, (const char *)s + i * sp, w);
-    return hipSuccess;
+    hipError_t e = hipSuccess;
+    for (size_t i = 0; i < h && e == hipSuccess; i++) e = hipMemcpy((char *)d + i * dp, (const char *)s + i * sp, w, k);
+    return e;
 }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { *f = *t = (size_t)288 << 30; return hipSuccess; }
 hipError_t hipSetDevice(int d) { return d == 0 ? hipSuccess : (last = hipErrorInvalidDevice); }

@@ -329,3 +329,34 @@ def test_an_adjoint_that_gave_up_is_not_tried_again(stub, monkeypatch, capfd):
         _grad(m, 9)                                  # the forward loop did get on
         assert stub.get("resident") == 2 and stub.get("adjoint") == 2
     assert "resident adjoint off" in capfd.readouterr().err
+
+
+@pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
+def test_no_call_needs_the_legacy_stream(kind, stub):
+    """hipMemcpy fails, and spoils the capture, while another thread captures a
+    graph: handles of other threads must get on without it."""
+    stub.set("capturing", 1)
+    with _model(kind=kind) as m:
+        m.run(jsnap=2, snapshots=True)
+        m.run()
+        m.traces()
+        m.field()
+        if kind == "spher2d":
+            return
+        _grad(m, 9)
+        _grad(m, 3)
+    m = _model(kind=kind, cden=False)
+    m.set_model(np.full((40, 30), 1.7e8, np.float32), np.full((40, 30), 900.0, np.float32))
+    m.run()
+    ms = [_model(nt=30) for _ in range(2)]
+    b = awefd.Batch(ms)
+    res, rp = _dev(30, 5)
+    g, gp = _dev(40, 30)
+    for depth in (1, 2, 3):
+        b.set_tile(8)
+        b.set_depth(depth)
+        b.run()
+        for ckpt in (0, 30, 4):
+            b.run_ckpt(ckpt)
+            b.adjoint_grad([rp, rp], gp)
+    b.close()

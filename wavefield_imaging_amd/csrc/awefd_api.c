@@ -328,6 +328,16 @@ int awefd_padded_dims(const awefd_model *m, int dims[3], int *nb)
 
 int awefd_device(const awefd_model *m) { return m ? m->dev : -1; }
 
+/* A copy that has ended when it returns, after the legacy stream's work as
+ * hipMemcpy orders it, on the caller's own stream: hipMemcpy itself fails while
+ * another thread captures a graph, and spoils that capture. */
+hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t stream)
+{
+    hipError_t e = hipStreamSynchronize(NULL);
+    if (e == hipSuccess) e = hipMemcpyAsync(dst, src, n, kind, stream);
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+}
+
 /* Rows between dense host memory and device rows of dpitch bytes.  A 2-D copy
  * of pageable memory goes row by row (7 us each: 3.2 ms for the 467 rows of a
  * 271 x 467 field, 9 ms for its velocity and density records), so the rows
@@ -336,19 +346,21 @@ int awefd_device(const awefd_model *m) { return m ? m->dev : -1; }
  * as zero on the way up. */
 #define ROWS_STAGE ((size_t)16 << 20)
 
-static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, size_t nrows, int up)
+static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, size_t nrows, int up, hipStream_t stream)
 {
     if (!nrows || !row) return hipSuccess;
     if (dpitch == row)
-        return hipMemcpy(up ? dev : host, up ? host : dev, row * nrows, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
+        return awefd__copy(up ? dev : host, up ? host : dev, row * nrows,
+                           up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, stream);
     size_t per = ROWS_STAGE / dpitch;
     if (per < 1) per = 1;
     if (per > nrows) per = nrows;
     char *st = malloc(per * dpitch);
-    if (!st)                             /* no staging: the copy of single rows */
-        return up ? hipMemcpy2D(dev, dpitch, host, row, row, nrows, hipMemcpyHostToDevice)
-                  : hipMemcpy2D(host, row, dev, dpitch, row, nrows, hipMemcpyDeviceToHost);
     hipError_t e = hipSuccess;
+    for (size_t r = 0; !st && r < nrows && e == hipSuccess; r++)         /* no staging: single rows */
+        e = up ? awefd__copy(dev + r * dpitch, host + r * row, row, hipMemcpyHostToDevice, stream)
+               : awefd__copy(host + r * row, dev + r * dpitch, row, hipMemcpyDeviceToHost, stream);
+    if (!st) return e;
     for (size_t r0 = 0; r0 < nrows && e == hipSuccess; r0 += per) {
         const size_t n = nrows - r0 < per ? nrows - r0 : per;
         if (up) {
@@ -356,9 +368,9 @@ static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, si
                 memcpy(st + r * dpitch, host + (r0 + r) * row, row);
                 memset(st + r * dpitch + row, 0, dpitch - row);
             }
-            e = hipMemcpy(dev + r0 * dpitch, st, n * dpitch, hipMemcpyHostToDevice);
+            e = awefd__copy(dev + r0 * dpitch, st, n * dpitch, hipMemcpyHostToDevice, stream);
         } else {
-            e = hipMemcpy(st, dev + r0 * dpitch, n * dpitch, hipMemcpyDeviceToHost);
+            e = awefd__copy(st, dev + r0 * dpitch, n * dpitch, hipMemcpyDeviceToHost, stream);
             for (size_t r = 0; e == hipSuccess && r < n; r++) memcpy(host + (r0 + r) * row, st + r * dpitch, row);
         }
     }
@@ -366,14 +378,14 @@ static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, si
     return e;
 }
 
-hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows)
+hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows, hipStream_t stream)
 {
-    return rows_copy(dev, dpitch, (char *)(uintptr_t)host, row, nrows, 1);
+    return rows_copy(dev, dpitch, (char *)(uintptr_t)host, row, nrows, 1, stream);
 }
 
-hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows)
+hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows, hipStream_t stream)
 {
-    return rows_copy((char *)(uintptr_t)dev, dpitch, host, row, nrows, 0);
+    return rows_copy((char *)(uintptr_t)dev, dpitch, host, row, nrows, 0, stream);
 }
 
 static int upload(awefd_model *m, void **dst, const void *src, size_t bytes)
@@ -381,8 +393,7 @@ static int upload(awefd_model *m, void **dst, const void *src, size_t bytes)
     free_dev(dst);
     if (bytes == 0) return AWEFD_OK;
     HIPCHK(hipMalloc(dst, bytes));
-    HIPCHK(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
-    (void)m;
+    HIPCHK(awefd__copy(*dst, src, bytes, hipMemcpyHostToDevice, m->stream));
     return AWEFD_OK;
 }
 
@@ -424,7 +435,7 @@ static int cart_set_density(awefd_model *m, const float *den)
     free_dev((void **)&m->drho);
     hipError_t e = hipMalloc((void **)&m->drho, sizeof(float) * 4 * (size_t)m->nalloc);
     if (e == hipSuccess)
-        e = awefd__rows_up(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, (size_t)n2 * n3);
+        e = awefd__rows_up(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, (size_t)n2 * n3, m->stream);
     free(g);
     if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "density upload: %s", hipGetErrorString(e));
     return AWEFD_OK;
@@ -512,7 +523,7 @@ static int cart_set_model(awefd_model *m, const float *vel, const float *den)
         for (long c = 0; c < (long)n2 * n3; c++)
             for (int iz = 0; iz <= m->nb && iz < n1; iz++) v[c * n1 + iz] = 0.f;
     if (rc == 0) {
-        hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1, (size_t)n2 * n3);
+        hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1, (size_t)n2 * n3, m->stream);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "vel upload: %s", hipGetErrorString(e));
     }
     free(v);
@@ -870,7 +881,8 @@ static int prof_collect(awefd_model *m, int npairs)
 /* Device field (row stride ld) to a dense host array (row stride np[0]). */
 static hipError_t copy_field_out(const awefd_model *m, float *host, const float *dev)
 {
-    return awefd__rows_down(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2]);
+    return awefd__rows_down(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2],
+                            m->stream);
 }
 
 /* Apply the pending sponge factor to a host copy of the stored field (the
@@ -1158,8 +1170,8 @@ int awefd_run(awefd_model *m, float *traces, int jsnap, awefd_snap_fn cb, void *
     int rc = run_common(m, NULL, jsnap, cb, user);
     if (rc) return rc;
     if (traces && m->nr > 0 && !m->adj2)
-        HIPCHK(hipMemcpy(traces, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr,
-                         hipMemcpyDeviceToHost));
+        HIPCHK(awefd__copy(traces, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost,
+                           m->stream));
     return AWEFD_OK;
 }
 
@@ -1203,7 +1215,7 @@ int awefd_get_traces(awefd_model *m, float *host)
     HIPCHK(hipSetDevice(m->dev));
     HIPCHK(hipStreamSynchronize(m->stream));
     if (m->nr > 0)
-        HIPCHK(hipMemcpy(host, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost));
+        HIPCHK(awefd__copy(host, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost, m->stream));
     return AWEFD_OK;
 }
 
