@@ -1,6 +1,9 @@
 """Handles of several threads at once on one GPU: resident loops (cartesian,
 polar, a gradient) beside each other, beside a loop and batches that capture
 graphs, and beside set-ups; each gives what it gives alone, bit for bit."""
+import os
+import subprocess
+import sys
 import threading
 import traceback
 
@@ -89,3 +92,37 @@ def test_handles_of_several_threads(monkeypatch, capfd):
     assert not bad, bad
     err = capfd.readouterr().err
     assert "resident 2-D loop" in err and "resident adjoint" in err and "off" not in err
+
+
+CHILD = """
+import sys
+sys.path[:0] = [%r, %r]
+import numpy as np
+import test_gpu_kept_fields as kept
+import test_gpu_resident as cart
+import test_gpu_resident_polar as polar
+import test_gpu_threads as t
+for k, run in enumerate((t._forward("cart2d", cart._case(83, 130, 9, 150, 1)[:5]),
+                         t._forward("spher2d", polar._case(150, 210, 9, 150)), t._gradient(kept._case(97, 203, 80, 12)))):
+    for _ in range(3):
+        out = run()
+    np.save(sys.argv[1] + "/%%d.npy" %% k, out)
+    print("case", k, flush=True)
+"""
+
+
+def test_a_second_process(tmp_path):
+    """One process at a time has a card's cooperative queue: beside one that
+    runs resident loops, another runs the loops of one launch per step, and
+    gives the same."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    runs = [_forward("cart2d", cart._case(83, 130, 9, 150, 1)[:5]), _forward("spher2d", polar._case(150, 210, 9, 150)),
+            _gradient(kept._case(97, 203, 80, 12))]
+    want = [r() for r in runs]
+    child = subprocess.Popen([sys.executable, "-c", CHILD % (os.path.dirname(here), here), str(tmp_path)])
+    while child.poll() is None:                          # this process's runs go on beside it
+        for r, w in zip(runs, want):
+            np.testing.assert_array_equal(r(), w)
+    assert child.returncode == 0
+    for k, w in enumerate(want):
+        np.testing.assert_array_equal(np.load(tmp_path / ("%d.npy" % k)), w)

@@ -269,8 +269,9 @@ def test_shots_of_a_batch_hold_no_rims(stub, monkeypatch):
 @pytest.mark.parametrize("kind", ["cart2d", "spher2d"])
 def test_launch_errors_of_a_resident_loop(kind, stub):
     """A device that cannot hold the blocks (720) or launch them together
-    (801): the other loop, from then on.  Any other error is the run's."""
-    for code in (720, 801):
+    (801), or whose cooperative queue another process has (401): the other
+    loop, from then on.  A failed device or kernel is the run's error."""
+    for code in (720, 801, 401):
         with _model(kind=kind) as m:
             stub.reset()
             stub.set("launch_error", code)

@@ -480,7 +480,7 @@ static int resadj_run(awefd_model *m, adj_state *s, const awefd_adj2d_args *g, i
     const int l = awefd__resadj_launch(&a, a.ntz * a.ntx, m->nop, s->rt.rx, m->stream);
     if (l) {
         (void)hipGetLastError();
-        if (!awefd__res_refused(l))
+        if (awefd__res_broken(l))
             return awefd__fail(AWEFD_EHIP, "resident adjoint: %s", hipGetErrorString((hipError_t)l));
         awefd__res_off(&s->rt.on, "adjoint", hipGetErrorString((hipError_t)l));
         return AWEFD_OK;

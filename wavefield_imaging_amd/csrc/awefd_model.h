@@ -156,7 +156,7 @@ int  awefd__res_buffers(awefd_model *m);
 int  awefd__res_flag(awefd_model *m);
 void awefd__res_prepare(awefd_model *m);
 void awefd__res_wait(unsigned *wmask, long long *wticks);
-int  awefd__res_refused(int e);
+int  awefd__res_broken(int e);
 void awefd__res_off(int *on, const char *who, const char *why);
 int  awefd__res_finish(awefd_model *m, int launched, int *done);
 /* resident polar loop (spher_host.c) */

@@ -329,12 +329,15 @@ void awefd__res_args(const awefd_model *m, const awefd_res_tile *t, const awefd_
     awefd__res_wait(&a->wmask, &a->wticks);
 }
 
-/* Whether a cooperative launch was refused for what the device can hold or do
- * (the caller then has another loop), not for an error of its own. */
-int awefd__res_refused(int e)
+/* Whether a launch error is a failure of the device or of an earlier kernel.
+ * Every other one is the cooperative launch's refusal, for which the caller has
+ * another loop: too many blocks, not supported, or (hipErrorIllegalState) a
+ * second process on a card, one process at a time having its cooperative queue. */
+int awefd__res_broken(int e)
 {
-    return e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported || e == hipErrorInvalidConfiguration ||
-           e == hipErrorInvalidValue || e == hipErrorLaunchOutOfResources || e == hipErrorOutOfMemory;
+    return e == hipErrorIllegalAddress || e == hipErrorLaunchFailure || e == hipErrorLaunchTimeOut ||
+           e == hipErrorAssert || e == hipErrorECCNotCorrectable || e == hipErrorNoDevice ||
+           e == hipErrorInvalidContext || e == hipErrorContextIsDestroyed;
 }
 
 /* The resident loop `who` is not tried again by this handle: *on = 0. */
@@ -351,7 +354,7 @@ int awefd__res_finish(awefd_model *m, int launched, int *done)
     awefd_res *r = &m->res;
     if (launched) {
         (void)hipGetLastError();
-        if (!awefd__res_refused(launched))
+        if (awefd__res_broken(launched))
             return awefd__fail(AWEFD_EHIP, "resident loop: %s", hipGetErrorString((hipError_t)launched));
         awefd__res_off(&r->on, "loop", hipGetErrorString((hipError_t)launched));
         return AWEFD_OK;
