@@ -29,9 +29,10 @@ Roofline: algorithmic bytes (16 per node update: read the previous field, the
 current field and the velocity term, write the new field) over the dominant
 kernel's time.  3-D: the kernel's mean duration from HIP events around every
 launch on its own stream, inside the timed region.  cart2d runs as one
-launch per shot that keeps the fields on the chip: its time per step over the
-timed region, with the same 16 bytes per node update (none of which reach HBM,
-so its "frac" is a rate, not a share of a limit).  batch2d and adjoint2d run as
+launch per shot that keeps the fields on the chip, so it moves none of these
+bytes and has no share of the HBM limit ("achieved" and "frac" are null; its
+bound is the latency of the exchange between blocks); its kernel time is the
+time per step over the timed region.  batch2d and adjoint2d run as
 graphs: real bytes of their passes over the timed graphs (20 bytes per
 node for a three-step pass; for a gradient the bytes of its forward,
 checkpoint, recompute and adjoint passes, 32.9 per node and step with
@@ -219,13 +220,15 @@ def measure(workload, nt, steps, warmup):
         timing = "one launch per shot, fields on the chip: time per step over the timed shots"
     m.profile(False)
     m.close()
-    achieved = BYTES_PER_UPDATE * cells / (avg_ms * 1e-3) / 1e9
+    achieved = BYTES_PER_UPDATE * cells / (avg_ms * 1e-3) / 1e9 if eager_timed else None
     out = dict(workload=w["desc"] % nt, cells_per_step=cells, time_steps_per_shot=nt,
                value=round(cells * nt * steps / secs / 1e9, 3),
                ms_per_step=round(secs / steps * 1e3, 3),
                ms_per_time_step=round(secs / steps / nt * 1e3, 5),
-               roofline={"bound": "hbm" if eager_timed else "latency", "achieved": round(achieved, 1),
-                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+               roofline={"bound": "hbm" if eager_timed else "latency",
+                         "achieved": round(achieved, 1) if eager_timed else None,
+                         "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                         "frac": round(achieved / HBM_PEAK_GBS, 4) if eager_timed else None,
                          "traffic": _traffic(w["traffic"]), "kernel": w["kernel"],
                          "kernel_mean_ms": round(avg_ms, 5), "launches": launches, "timing": timing})
     return out, case

@@ -4,8 +4,12 @@
  *
  * A cartesian model takes it when it is 2-D in the SSE order with fdorder up
  * to 8, bilinear points, no hybrid boundary, and a compiled tile whose blocks
- * are at most the CUs.  Profiled runs, runs with snapshots and
- * awefd_run_noalloc keep the loop of one launch per step.  AWEFD_RESIDENT=0
+ * are at most the CUs: at best 3.9 M padded nodes for fdorder 4 (3.7 M for 8),
+ * 0.86 M (0.69 M) with variable density, whose records leave registers for at
+ * most 4 rows a wave.  Profiled runs, runs with snapshots and
+ * awefd_run_noalloc keep the loop of one launch per step, and so do all runs
+ * of a second process on a card, whose cooperative queue has one process at a
+ * time.  AWEFD_RESIDENT=0
  * turns it off for the models created after, AWEFD_RES_STEPS=1 or 2 asks for
  * that many steps per exchange.
  */

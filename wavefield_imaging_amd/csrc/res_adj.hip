@@ -8,7 +8,9 @@
  * Infinity Cache, but as a launch it took 7.6 us, most of it the latency of
  * its loads.  Here alpha_{n+1}, alpha_{n+2}, V and dJ/dV stay in registers,
  * y = V M G alpha_{n+1} in LDS, whose rim is all the neighbours need, and only
- * c_n is read, a step ahead: 2.9 us a step.
+ * c_n is read, a step ahead: 2.9 us a step.  Up to 12 rows a wave fit the
+ * registers with fdorder 2 and 4 (1.5 M padded nodes at best), 10 with 6
+ * (1.2 M) and 8 with 8 (0.9 M); larger grids keep a launch per step.
  *
  * Arithmetic, order and selections are adj_body's (adj_kernels.hip) node for
  * node: the same bits.

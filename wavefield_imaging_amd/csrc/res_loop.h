@@ -14,7 +14,8 @@
  *
  * Rim exchange.  A rim value travels as one 64-bit word {tag, value}, stored
  * and polled with device-scope relaxed atomics (8 bytes, so value and tag
- * arrive together: no separate flag, no fence, no wait for the stores).
+ * arrive together: no separate flag and no fence; the poll's own wait covers
+ * the stores issued before it, which share its counter).
  * Alone, one exchange between 8 to 256 blocks takes 0.75-0.95 us (64 words a
  * side), whichever XCDs the neighbours sit on.  Words are double-buffered by
  * the parity of the exchange: a block overwrites exchange e's words at
@@ -29,13 +30,16 @@
  *
  * S steps per exchange: the tile carries a margin of S NOP nodes on every
  * side; each step consumes NOP of it, and the blocks compute the margin's
- * inner nodes redundantly.  S = 2 halves the exchanges for 4 NOP more nodes
- * a side; the chip holds fewer owned nodes, so the largest grids run S = 1.
+ * inner nodes redundantly.  S = 2 halves the exchanges for a margin of 2 NOP
+ * nodes a side instead of NOP (S NOP in general, (S - 1) NOP of them
+ * computed); the chip holds fewer owned nodes, so the largest grids run S = 1.
+ * More than two steps an exchange were not built.
  *
  * Progress.  The launch is cooperative: all blocks are resident before any
  * runs.  A wait is bounded all the same: after 4 s without its words (or
  * once another block has given up) a block raises the stop flag and leaves;
- * the host then runs the one-launch-per-step loop instead.
+ * the host then runs the one-launch-per-step loop instead, from then on for
+ * that handle.
  *
  * Tile.  A wave holds 64 z lanes, the outer S NOP on each side the margin,
  * of RX x rows; 16 waves a block with S = 2 (4 per SIMD, up to 96 rows: the
@@ -211,7 +215,7 @@ __global__ __launch_bounds__(nwave(S) * WAVE) void k_cart2d_res(const awefd_res_
         const bool in = ix >= 0 && ix < n2;
         V[j] = bld(rV, in ? vz : OOB, in ? (unsigned)ix * rowb : 0u);
         if (VD) {
-            /* 1 beyond the grid: its lanes divide too */
+            /* 0 beyond the grid: the quotient there is NaN, and masked */
             const unsigned vg = in && zin ? (unsigned)iz * 16u : OOB, sg = in ? 4u * (unsigned)ix * rowb : 0u;
             g[j] = make_float4(bld(rR, vg, sg), bld(rR, vg + 4u, sg), bld(rR, vg + 8u, sg), bld(rR, vg + 12u, sg));
         }
@@ -350,8 +354,8 @@ __global__ __launch_bounds__(nwave(S) * WAVE) void k_cart2d_res(const awefd_res_
                 }
             amp = na;
         }
-        /* the gradient keeps every field: the owned nodes, stored and not
-         * waited for */
+        /* the gradient keeps every field: the owned nodes (the next poll's
+         * wait covers the stores) */
         if (__builtin_expect(a.F != nullptr, 0) && it + 1 < nt) {
             const rsrc_t rF = mk_rsrc(a.F + (long)it * a.nal, (unsigned)n2 * rowb);
 #pragma unroll

@@ -20,7 +20,9 @@
  * crosses the two theta lines is that neighbour one whose own rule comes
  * first in the sweep, and its value the final one.  So a chain has at most
  * two levels, inside the tile when the tiles at the high faces own
- * AWEFD_POLAR_FACE nodes (the host picks such a tile).  The host lists the
+ * AWEFD_POLAR_FACE nodes (the host picks such a tile; padded r of 63-67, 125-127,
+ * 187 and some above 1,680 nodes leave the last tile of both widths, 62 and 60,
+ * with fewer, and keep the loop of several launches per step).  The host lists the
  * nodes per block, two a thread: the values before the boundary go to the
  * image, a barrier, the listed nodes are evaluated, a barrier, the final
  * values replace them.  Blocks without such nodes store final values at once.
