@@ -79,6 +79,7 @@ hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, s
 }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { *f = *t = (size_t)288 << 30; return hipSuccess; }
 hipError_t hipSetDevice(int d) { return d == 0 ? hipSuccess : (last = hipErrorInvalidDevice); }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d)
 {
     (void)d;

@@ -145,9 +145,9 @@ static int point_buckets(const awefd_model *m, int n, const int *j, const float 
         awefd_sort_inj(keys, ne, nbucket, e, beg);
         hipError_t er = hipMalloc((void **)d_inj, sizeof(*e) * (ne > 0 ? ne : 1));
         if (er == hipSuccess) er = hipMalloc((void **)d_beg, sizeof(int) * (nbucket + 1));
-        if (er == hipSuccess && ne) er = awefd__copy(*d_inj, e, sizeof(*e) * ne, hipMemcpyHostToDevice, m->stream);
+        if (er == hipSuccess && ne) er = awefd__copy(*d_inj, e, sizeof(*e) * ne, hipMemcpyHostToDevice);
         if (er == hipSuccess)
-            er = awefd__copy(*d_beg, beg, sizeof(int) * (nbucket + 1), hipMemcpyHostToDevice, m->stream);
+            er = awefd__copy(*d_beg, beg, sizeof(int) * (nbucket + 1), hipMemcpyHostToDevice);
         if (er != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "gradient point buckets: %s", hipGetErrorString(er));
     }
     free(keys); free(e); free(beg);
@@ -634,7 +634,7 @@ int awefd_adjoint_grad(awefd_model *m, const float *d_res, float *d_grad)
     awefd_adj2d_args g;
     if ((rc = awefd__adj_prepare(m))) goto done;
     awefd__adj_args(m, d_res, &g);
-    HIPCHK(awefd__copy(s->d_args, &g, sizeof g, hipMemcpyHostToDevice, m->stream));
+    HIPCHK(awefd__copy(s->d_args, &g, sizeof g, hipMemcpyHostToDevice));
     int done = 0;
     if (s->kept && (rc = resadj_run(m, s, &g, &done))) goto done;
     if (!done) {

@@ -10,6 +10,7 @@
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
 #include <math.h>
+#include <pthread.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -328,12 +329,29 @@ int awefd_padded_dims(const awefd_model *m, int dims[3], int *nb)
 
 int awefd_device(const awefd_model *m) { return m ? m->dev : -1; }
 
-/* A copy that has ended when it returns, after the legacy stream's work as
- * hipMemcpy orders it, on the caller's own stream: hipMemcpy itself fails while
- * another thread captures a graph, and spoils that capture. */
-hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t stream)
+/* A device's stream for copies, made by its first one and kept like the
+ * runtime's own null stream (a stream's first use takes half a millisecond: 60
+ * shots of a batch, copied to on a stream of each, took 34 ms longer to set
+ * up). */
+#define COPY_MAX_DEV 64
+static hipStream_t copy_stream[COPY_MAX_DEV];
+static pthread_mutex_t copy_lock = PTHREAD_MUTEX_INITIALIZER;
+
+/* A copy that has ended when it returns, after the legacy stream's work, as
+ * hipMemcpy does it; but hipMemcpy fails while another thread captures a graph,
+ * and spoils that capture. */
+hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind)
 {
-    hipError_t e = hipStreamSynchronize(NULL);
+    int dev = -1;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= COPY_MAX_DEV) return hipErrorInvalidDevice;
+    pthread_mutex_lock(&copy_lock);
+    if (!copy_stream[dev]) e = hipStreamCreateWithFlags(&copy_stream[dev], hipStreamNonBlocking);
+    if (e != hipSuccess) copy_stream[dev] = NULL;
+    const hipStream_t stream = copy_stream[dev];
+    pthread_mutex_unlock(&copy_lock);
+    if (e == hipSuccess) e = hipStreamSynchronize(NULL);
     if (e == hipSuccess) e = hipMemcpyAsync(dst, src, n, kind, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
 }
@@ -346,20 +364,19 @@ hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind,
  * as zero on the way up. */
 #define ROWS_STAGE ((size_t)16 << 20)
 
-static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, size_t nrows, int up, hipStream_t stream)
+static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, size_t nrows, int up)
 {
     if (!nrows || !row) return hipSuccess;
     if (dpitch == row)
-        return awefd__copy(up ? dev : host, up ? host : dev, row * nrows,
-                           up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, stream);
+        return awefd__copy(up ? dev : host, up ? host : dev, row * nrows, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
     size_t per = ROWS_STAGE / dpitch;
     if (per < 1) per = 1;
     if (per > nrows) per = nrows;
     char *st = malloc(per * dpitch);
     hipError_t e = hipSuccess;
     for (size_t r = 0; !st && r < nrows && e == hipSuccess; r++)         /* no staging: single rows */
-        e = up ? awefd__copy(dev + r * dpitch, host + r * row, row, hipMemcpyHostToDevice, stream)
-               : awefd__copy(host + r * row, dev + r * dpitch, row, hipMemcpyDeviceToHost, stream);
+        e = up ? awefd__copy(dev + r * dpitch, host + r * row, row, hipMemcpyHostToDevice)
+               : awefd__copy(host + r * row, dev + r * dpitch, row, hipMemcpyDeviceToHost);
     if (!st) return e;
     for (size_t r0 = 0; r0 < nrows && e == hipSuccess; r0 += per) {
         const size_t n = nrows - r0 < per ? nrows - r0 : per;
@@ -368,9 +385,9 @@ static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, si
                 memcpy(st + r * dpitch, host + (r0 + r) * row, row);
                 memset(st + r * dpitch + row, 0, dpitch - row);
             }
-            e = awefd__copy(dev + r0 * dpitch, st, n * dpitch, hipMemcpyHostToDevice, stream);
+            e = awefd__copy(dev + r0 * dpitch, st, n * dpitch, hipMemcpyHostToDevice);
         } else {
-            e = awefd__copy(st, dev + r0 * dpitch, n * dpitch, hipMemcpyDeviceToHost, stream);
+            e = awefd__copy(st, dev + r0 * dpitch, n * dpitch, hipMemcpyDeviceToHost);
             for (size_t r = 0; e == hipSuccess && r < n; r++) memcpy(host + (r0 + r) * row, st + r * dpitch, row);
         }
     }
@@ -378,14 +395,14 @@ static hipError_t rows_copy(char *dev, size_t dpitch, char *host, size_t row, si
     return e;
 }
 
-hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows, hipStream_t stream)
+hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows)
 {
-    return rows_copy(dev, dpitch, (char *)(uintptr_t)host, row, nrows, 1, stream);
+    return rows_copy(dev, dpitch, (char *)(uintptr_t)host, row, nrows, 1);
 }
 
-hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows, hipStream_t stream)
+hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows)
 {
-    return rows_copy((char *)(uintptr_t)dev, dpitch, host, row, nrows, 0, stream);
+    return rows_copy((char *)(uintptr_t)dev, dpitch, host, row, nrows, 0);
 }
 
 static int upload(awefd_model *m, void **dst, const void *src, size_t bytes)
@@ -393,7 +410,8 @@ static int upload(awefd_model *m, void **dst, const void *src, size_t bytes)
     free_dev(dst);
     if (bytes == 0) return AWEFD_OK;
     HIPCHK(hipMalloc(dst, bytes));
-    HIPCHK(awefd__copy(*dst, src, bytes, hipMemcpyHostToDevice, m->stream));
+    HIPCHK(awefd__copy(*dst, src, bytes, hipMemcpyHostToDevice));
+    (void)m;
     return AWEFD_OK;
 }
 
@@ -435,7 +453,7 @@ static int cart_set_density(awefd_model *m, const float *den)
     free_dev((void **)&m->drho);
     hipError_t e = hipMalloc((void **)&m->drho, sizeof(float) * 4 * (size_t)m->nalloc);
     if (e == hipSuccess)
-        e = awefd__rows_up(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, (size_t)n2 * n3, m->stream);
+        e = awefd__rows_up(m->drho, sizeof(float) * 4 * m->ld, g, sizeof(float) * 4 * n1, (size_t)n2 * n3);
     free(g);
     if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "density upload: %s", hipGetErrorString(e));
     return AWEFD_OK;
@@ -523,7 +541,7 @@ static int cart_set_model(awefd_model *m, const float *vel, const float *den)
         for (long c = 0; c < (long)n2 * n3; c++)
             for (int iz = 0; iz <= m->nb && iz < n1; iz++) v[c * n1 + iz] = 0.f;
     if (rc == 0) {
-        hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1, (size_t)n2 * n3, m->stream);
+        hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, v, sizeof(float) * n1, (size_t)n2 * n3);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "vel upload: %s", hipGetErrorString(e));
     }
     free(v);
@@ -881,8 +899,7 @@ static int prof_collect(awefd_model *m, int npairs)
 /* Device field (row stride ld) to a dense host array (row stride np[0]). */
 static hipError_t copy_field_out(const awefd_model *m, float *host, const float *dev)
 {
-    return awefd__rows_down(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2],
-                            m->stream);
+    return awefd__rows_down(host, sizeof(float) * m->np[0], dev, sizeof(float) * m->ld, (size_t)m->np[1] * m->np[2]);
 }
 
 /* Apply the pending sponge factor to a host copy of the stored field (the
@@ -1170,8 +1187,7 @@ int awefd_run(awefd_model *m, float *traces, int jsnap, awefd_snap_fn cb, void *
     int rc = run_common(m, NULL, jsnap, cb, user);
     if (rc) return rc;
     if (traces && m->nr > 0 && !m->adj2)
-        HIPCHK(awefd__copy(traces, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost,
-                           m->stream));
+        HIPCHK(awefd__copy(traces, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost));
     return AWEFD_OK;
 }
 
@@ -1215,7 +1231,7 @@ int awefd_get_traces(awefd_model *m, float *host)
     HIPCHK(hipSetDevice(m->dev));
     HIPCHK(hipStreamSynchronize(m->stream));
     if (m->nr > 0)
-        HIPCHK(awefd__copy(host, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost, m->stream));
+        HIPCHK(awefd__copy(host, m->d_traces, sizeof(float) * (size_t)m->p.nt * m->nr, hipMemcpyDeviceToHost));
     return AWEFD_OK;
 }
 

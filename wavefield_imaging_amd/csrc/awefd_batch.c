@@ -119,9 +119,9 @@ static void dfree(void *pp)
     *p = NULL;
 }
 
-static hipError_t up(const awefd_batch *b, void *dst, const void *src, size_t n)
+static hipError_t up(void *dst, const void *src, size_t n)
 {
-    return awefd__copy(dst, src, n, hipMemcpyHostToDevice, b->stream);
+    return awefd__copy(dst, src, n, hipMemcpyHostToDevice);
 }
 
 void awefd_batch_destroy(awefd_batch *b)
@@ -309,8 +309,8 @@ static int batch_build(awefd_batch *b, int rx, int group_mb)
             hipError_t e = hipMalloc((void **)&b->d_inj[s], sizeof(*inj) * (ninj > 0 ? ninj : 1));
             if (e == hipSuccess) e = hipMalloc((void **)&b->d_ibeg[s], sizeof(int) * (nbucket + 1));
             if (e == hipSuccess && ninj > 0)
-                e = up(b, b->d_inj[s], inj, sizeof(*inj) * ninj);
-            if (e == hipSuccess) e = up(b, b->d_ibeg[s], ibeg, sizeof(int) * (nbucket + 1));
+                e = up(b->d_inj[s], inj, sizeof(*inj) * ninj);
+            if (e == hipSuccess) e = up(b->d_ibeg[s], ibeg, sizeof(int) * (nbucket + 1));
             if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "batch injection upload: %s", hipGetErrorString(e));
             h[s].inj = b->d_inj[s];
             h[s].ibeg = b->d_ibeg[s];
@@ -329,8 +329,8 @@ static int batch_build(awefd_batch *b, int rx, int group_mb)
         dfree(&b->d_bshot);
         hipError_t e = hipMalloc((void **)&b->d_shots, sizeof(*h) * b->nshot);
         if (e == hipSuccess) e = hipMalloc((void **)&b->d_bshot, sizeof(int) * total);
-        if (e == hipSuccess) e = up(b, b->d_shots, h, sizeof(*h) * b->nshot);
-        if (e == hipSuccess) e = up(b, b->d_bshot, bshot, sizeof(int) * total);
+        if (e == hipSuccess) e = up(b->d_shots, h, sizeof(*h) * b->nshot);
+        if (e == hipSuccess) e = up(b->d_bshot, bshot, sizeof(int) * total);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "batch table upload: %s", hipGetErrorString(e));
     }
     free(bshot);
@@ -578,8 +578,8 @@ static int t2_build(awefd_batch *b, int depth)
             dfree(&b->d_ibeg2[s]);
             e = hipMalloc((void **)&b->d_inj2[s], sizeof(*inj) * (ninj > 0 ? ninj : 1));
             if (e == hipSuccess) e = hipMalloc((void **)&b->d_ibeg2[s], sizeof(int) * (h->nblk2 + 1));
-            if (e == hipSuccess && ninj > 0) e = up(b, b->d_inj2[s], inj, sizeof(*inj) * ninj);
-            if (e == hipSuccess) e = up(b, b->d_ibeg2[s], ibeg, sizeof(int) * (h->nblk2 + 1));
+            if (e == hipSuccess && ninj > 0) e = up(b->d_inj2[s], inj, sizeof(*inj) * ninj);
+            if (e == hipSuccess) e = up(b->d_ibeg2[s], ibeg, sizeof(int) * (h->nblk2 + 1));
             if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "two-step injection upload: %s", hipGetErrorString(e));
             h->inj2 = b->d_inj2[s];
             h->ibeg2 = b->d_ibeg2[s];
@@ -598,8 +598,8 @@ static int t2_build(awefd_batch *b, int depth)
                 const size_t nbeg = (size_t)h->ntz2 * h->ntx2 + 1, nrl = m->nr > 0 ? m->nr : 1;
                 e = hipMalloc((void **)&b->d_rbeg3[s], sizeof(int) * nbeg);
                 if (e == hipSuccess) e = hipMalloc((void **)&b->d_rx3[s], sizeof(awefd_rx3) * nrl);
-                if (e == hipSuccess) e = up(b, b->d_rbeg3[s], rbeg, sizeof(int) * nbeg);
-                if (e == hipSuccess) e = up(b, b->d_rx3[s], rx, sizeof(awefd_rx3) * nrl);
+                if (e == hipSuccess) e = up(b->d_rbeg3[s], rbeg, sizeof(int) * nbeg);
+                if (e == hipSuccess) e = up(b->d_rx3[s], rx, sizeof(awefd_rx3) * nrl);
                 if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "three-step receiver upload: %s", hipGetErrorString(e));
                 h->rbeg3 = b->d_rbeg3[s];
                 h->rx3 = b->d_rx3[s];
@@ -616,8 +616,8 @@ static int t2_build(awefd_batch *b, int depth)
     if (!rc) {
         dfree(&b->d_bshot2);
         hipError_t e = hipMalloc((void **)&b->d_bshot2, sizeof(int) * goff2[ng]);
-        if (e == hipSuccess) e = up(b, b->d_bshot2, bshot, sizeof(int) * goff2[ng]);
-        if (e == hipSuccess) e = up(b, b->d_shots, b->h, sizeof(*b->h) * ns);
+        if (e == hipSuccess) e = up(b->d_bshot2, bshot, sizeof(int) * goff2[ng]);
+        if (e == hipSuccess) e = up(b->d_shots, b->h, sizeof(*b->h) * ns);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "two-step table upload: %s", hipGetErrorString(e));
     }
     free(bshot);
@@ -729,8 +729,8 @@ static int final_jobs(awefd_batch *b, int fp, int fc, final_copies *f)
     f->nch = c;
     hipError_t e = hipMalloc((void **)&f->d_jobs, sizeof(*jobs) * f->njob);
     if (e == hipSuccess) e = hipMalloc((void **)&f->d_cbeg, sizeof(long) * f->njob);
-    if (e == hipSuccess) e = up(b, f->d_jobs, jobs, sizeof(*jobs) * f->njob);
-    if (e == hipSuccess) e = up(b, f->d_cbeg, cbeg, sizeof(long) * f->njob);
+    if (e == hipSuccess) e = up(f->d_jobs, jobs, sizeof(*jobs) * f->njob);
+    if (e == hipSuccess) e = up(f->d_cbeg, cbeg, sizeof(long) * f->njob);
     free(jobs);
     free(cbeg);
     if (e != hipSuccess) return awefd__fail(AWEFD_EHIP, "final copies: %s", hipGetErrorString(e));
@@ -1085,8 +1085,8 @@ static int ckpt_tables(awefd_batch *b, int depth)
     dfree(&b->d_cbeg);
     hipError_t e = hipMalloc((void **)&b->d_jobs, sizeof(*jobs) * njob);
     if (e == hipSuccess) e = hipMalloc((void **)&b->d_cbeg, sizeof(long) * njob);
-    if (e == hipSuccess) e = up(b, b->d_jobs, jobs, sizeof(*jobs) * njob);
-    if (e == hipSuccess) e = up(b, b->d_cbeg, cbeg, sizeof(long) * njob);
+    if (e == hipSuccess) e = up(b->d_jobs, jobs, sizeof(*jobs) * njob);
+    if (e == hipSuccess) e = up(b->d_cbeg, cbeg, sizeof(long) * njob);
     free(jobs);
     free(cbeg);
     free(b->joff);
@@ -1150,7 +1150,7 @@ static int run_kept(awefd_batch *b)
     int rc = AWEFD_OK;
     if (depth == 3 && (!b->t2_ok || b->t2_depth != 3) && (rc = t2_build(b, 3))) return rc;
     for (int s = 0; s < b->nshot; s++) awefd__adj_cart_ckpt(b->m[s], &b->h[s]);
-    HIPCHK(up(b, b->d_shots, b->h, sizeof(*b->h) * b->nshot));
+    HIPCHK(up(b->d_shots, b->h, sizeof(*b->h) * b->nshot));
     if (!(b->xfwd && b->fwd_ok && b->fwd_depth == depth)) {
         if (b->xfwd) hipGraphExecDestroy(b->xfwd);
         if (b->gfwd) hipGraphDestroy(b->gfwd);
@@ -1317,14 +1317,14 @@ static int adj_tables(awefd_batch *b, const float *const *d_res)
             if (e == hipSuccess) e = hipMalloc((void **)&b->d_zjobs, sizeof(*z) * 3 * ns);
             if (e == hipSuccess) e = hipMalloc((void **)&b->d_zcbeg, sizeof(long) * 3 * ns);
         }
-        if (e == hipSuccess) e = up(b, b->d_adj, ha, sizeof(*ha) * ns);
-        if (e == hipSuccess) e = up(b, b->d_abshot, bshot, sizeof(int) * agoff[ng]);
-        if (e == hipSuccess) e = up(b, b->d_abshot2, bshot2, sizeof(int) * agoff2[ng]);
-        if (e == hipSuccess) e = up(b, b->d_zjobs, z, sizeof(*z) * 3 * ns);
-        if (e == hipSuccess) e = up(b, b->d_zcbeg, zc, sizeof(long) * 3 * ns);
+        if (e == hipSuccess) e = up(b->d_adj, ha, sizeof(*ha) * ns);
+        if (e == hipSuccess) e = up(b->d_abshot, bshot, sizeof(int) * agoff[ng]);
+        if (e == hipSuccess) e = up(b->d_abshot2, bshot2, sizeof(int) * agoff2[ng]);
+        if (e == hipSuccess) e = up(b->d_zjobs, z, sizeof(*z) * 3 * ns);
+        if (e == hipSuccess) e = up(b->d_zcbeg, zc, sizeof(long) * 3 * ns);
         /* the recompute reads each shot's checkpoint and segment bases */
         for (int s = 0; s < ns; s++) awefd__adj_cart_ckpt(b->m[s], &b->h[s]);
-        if (e == hipSuccess) e = up(b, b->d_shots, b->h, sizeof(*b->h) * ns);
+        if (e == hipSuccess) e = up(b->d_shots, b->h, sizeof(*b->h) * ns);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "adjoint tables: %s", hipGetErrorString(e));
     }
     free(bshot);

@@ -131,9 +131,9 @@ int awefd__fail(int code, const char *fmt, ...);
 /* cartesian helpers shared with the batched path (awefd_api.c) */
 void awefd__cart_args(const awefd_model *m, awefd_cart_args *a);
 int  awefd__ensure_traces(awefd_model *m);
-hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t stream);
-hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows, hipStream_t stream);
-hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows, hipStream_t stream);
+hipError_t awefd__copy(void *dst, const void *src, size_t n, hipMemcpyKind kind);
+hipError_t awefd__rows_up(void *dev, size_t dpitch, const void *host, size_t row, size_t nrows);
+hipError_t awefd__rows_down(void *host, size_t row, const void *dev, size_t dpitch, size_t nrows);
 int  awefd__cart_buckets(const awefd_model *m, int tz, int ntz, int tx, awefd_inj **inj, int **ibeg,
                          int *nbucket, long *ninj);
 

@@ -212,7 +212,7 @@ int awefd__res_sources(awefd_model *m, const awefd_res_tile *t, awefd_res_buf *o
         for (int b = nb; b > 0; b--) beg[b] = beg[b - 1];
         beg[0] = 0;
         rc = awefd__res_grow(out, bytes);
-        hipError_t he = rc ? hipSuccess : awefd__copy(out->p, h, bytes, hipMemcpyHostToDevice, m->stream);
+        hipError_t he = rc ? hipSuccess : awefd__copy(out->p, h, bytes, hipMemcpyHostToDevice);
         if (he != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident source table: %s", hipGetErrorString(he));
         *inj_off = head;
     }
@@ -239,7 +239,7 @@ int awefd__res_receivers(awefd_model *m, const awefd_res_tile *t, awefd_res_buf 
     const size_t bytes = sizeof(int) * ((size_t)nb + 1 + (nr > 0 ? nr : 1));
     int rc = awefd__res_grow(out, bytes);
     if (!rc) {
-        hipError_t he = awefd__copy(out->p, h, bytes, hipMemcpyHostToDevice, m->stream);
+        hipError_t he = awefd__copy(out->p, h, bytes, hipMemcpyHostToDevice);
         if (he != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident receiver table: %s", hipGetErrorString(he));
     }
     *idx_off = sizeof(int) * ((size_t)nb + 1);

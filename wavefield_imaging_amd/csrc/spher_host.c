@@ -66,13 +66,13 @@ static void dfree(void *pp)
     *p = NULL;
 }
 
-static int up(awefd_model *m, void *dst, const void *src, size_t bytes)
+static int up(void *dst, const void *src, size_t bytes)
 {
     void **d = (void **)dst;
     dfree(d);
     if (!bytes) return AWEFD_OK;
     HIPCHK(hipMalloc(d, bytes));
-    HIPCHK(awefd__copy(*d, src, bytes, hipMemcpyHostToDevice, m->stream));
+    HIPCHK(awefd__copy(*d, src, bytes, hipMemcpyHostToDevice));
     return AWEFD_OK;
 }
 
@@ -225,10 +225,10 @@ int awefd__spher_create(awefd_model *m)
                 mt2[(long)ith * n1 + ir] = 1 / (r2 * sn * sn);
             }
         }
-        if (!rc) rc = up(m, &s->d_mr2, mr2, sizeof(float) * n1);
-        if (!rc) rc = up(m, &s->d_mr1, mr1, sizeof(float) * n1);
-        if (!rc) rc = up(m, &s->d_mt1, mt1, sizeof(double) * (size_t)n1 * n2);
-        if (!rc) rc = up(m, &s->d_mt2, mt2, sizeof(double) * (size_t)n1 * n2);
+        if (!rc) rc = up(&s->d_mr2, mr2, sizeof(float) * n1);
+        if (!rc) rc = up(&s->d_mr1, mr1, sizeof(float) * n1);
+        if (!rc) rc = up(&s->d_mt1, mt1, sizeof(double) * (size_t)n1 * n2);
+        if (!rc) rc = up(&s->d_mt2, mt2, sizeof(double) * (size_t)n1 * n2);
         free(mr2); free(mr1); free(mt1); free(mt2);
     } else {
         /* solve_2D (spher_utils.c:355-364): per-r coefficients in float */
@@ -242,7 +242,7 @@ int awefd__spher_create(awefd_model *m)
             pc[5 * ir + 3] = (1 / (ra * ra * dth * dth));
             pc[5 * ir + 4] = (-2 / (ra * ra * dth * dth));
         }
-        rc = up(m, &s->d_pc, pc, sizeof(float) * 5 * n1);
+        rc = up(&s->d_pc, pc, sizeof(float) * 5 * n1);
         free(pc);
     }
     if (rc) return rc;
@@ -252,7 +252,7 @@ int awefd__spher_create(awefd_model *m)
     double *damp = malloc(sizeof(double) * (nb + 1));
     if (!damp) return awefd__fail(AWEFD_ENOMEM, "sponge table");
     for (int i = 0; i <= nb; i++) damp[i] = awefd_spher_damp(i, nb);
-    rc = up(m, &m->d_damp, damp, sizeof(double) * (nb + 1));
+    rc = up(&m->d_damp, damp, sizeof(double) * (nb + 1));
     free(damp);
     return rc ? rc : polar_create(m);
 }
@@ -274,7 +274,7 @@ int awefd__spher_set_model(awefd_model *m, const float *vel)
     awefd_pad(vel, vp, m->p.n, nbs);
     const float dt = m->p.dt;
     for (long i = 0; i < nc; i++) vv[i] = (dt * dt) * (vp[i] * vp[i]);
-    hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, vv, sizeof(float) * n1, (size_t)n2 * n3, m->stream);
+    hipError_t e = awefd__rows_up(m->dvel, sizeof(float) * m->ld, vv, sizeof(float) * n1, (size_t)n2 * n3);
     free(vv);
     if (e != hipSuccess) {
         free(vp);
@@ -331,7 +331,7 @@ int awefd__spher_set_model(awefd_model *m, const float *vel)
     }
     m->res.one_ok = !rc && !polar_oneway(m, t);
     for (int i = 0; i < 6; i++) {
-        if (!rc) rc = up(m, &s->d_ow[i], t[i], sizeof(float) * sz[i]);
+        if (!rc) rc = up(&s->d_ow[i], t[i], sizeof(float) * sz[i]);
         free(t[i]);
     }
     free(s->h_velp);
@@ -362,7 +362,7 @@ int awefd__spher_set_receivers(awefd_model *m)
         h[3 * r + 1] = m->h_rj[3 * r];
         h[3 * r + 2] = m->ndim == 3 ? m->h_rj[3 * r + 2] : 0;
     }
-    int rc = up(m, &s->d_rrtp, h, sizeof(int) * 3 * (m->nr > 0 ? m->nr : 1));
+    int rc = up(&s->d_rrtp, h, sizeof(int) * 3 * (m->nr > 0 ? m->nr : 1));
     free(h);
     m->res.rec_ok = !rc && !polar_receivers(m);
     if (!rc && !s->inj_dirty && m->h_sj) build_conflicts(m);
@@ -397,7 +397,7 @@ static void build_conflicts(awefd_model *m)
         }
         if (hit) h[n++] = r;
     }
-    if (!up(m, &s->d_conf, h, sizeof(int) * n)) s->nconf = n;
+    if (!up(&s->d_conf, h, sizeof(int) * n)) s->nconf = n;
     free(h);
 }
 
@@ -495,9 +495,9 @@ static int build_injection(awefd_model *m)
     if (!rc) {
         ibeg[nn] = (int)n;
         s->ninode = nn;
-        rc = up(m, &s->d_inode, node, sizeof(long) * (nn > 0 ? nn : 1));
-        if (!rc) rc = up(m, &s->d_ibeg, ibeg, sizeof(int) * (nn + 1));
-        if (!rc) rc = up(m, &s->d_iw, iw, sizeof(float) * 2 * (n > 0 ? n : 1));
+        rc = up(&s->d_inode, node, sizeof(long) * (nn > 0 ? nn : 1));
+        if (!rc) rc = up(&s->d_ibeg, ibeg, sizeof(int) * (nn + 1));
+        if (!rc) rc = up(&s->d_iw, iw, sizeof(float) * 2 * (n > 0 ? n : 1));
         m->res.src_ok = !rc && !polar_sources(m, node, nn);
     }
     free(e); free(node); free(ibeg); free(iw);
@@ -696,7 +696,7 @@ static int polar_oneway(awefd_model *m, float *const t[4])
     char *h = polar_items(m, &r->t, t, &r->one_off, &bytes, &fits);
     if (!h) return awefd__fail(AWEFD_ENOMEM, "one-way nodes");
     int rc = awefd__res_grow(&r->one, bytes);
-    hipError_t e = rc ? hipSuccess : awefd__copy(r->one.p, h, bytes, hipMemcpyHostToDevice, m->stream);
+    hipError_t e = rc ? hipSuccess : awefd__copy(r->one.p, h, bytes, hipMemcpyHostToDevice);
     free(h);
     return rc || e == hipSuccess ? rc : awefd__fail(AWEFD_EHIP, "one-way nodes: %s", hipGetErrorString(e));
 }
@@ -737,7 +737,7 @@ static int polar_sources(awefd_model *m, const long *node, int n)
     if (!rc) {
         const size_t bytes = head + sizeof(int) * 2 * (size_t)(h[nblk] > 0 ? h[nblk] : 1);
         rc = awefd__res_grow(&r->src, bytes);
-        hipError_t e = rc ? hipSuccess : awefd__copy(r->src.p, h, bytes, hipMemcpyHostToDevice, m->stream);
+        hipError_t e = rc ? hipSuccess : awefd__copy(r->src.p, h, bytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident source table: %s", hipGetErrorString(e));
         r->inj_off = head;
     }
@@ -763,7 +763,7 @@ static int polar_receivers(awefd_model *m)
     for (int i = 0; i < nr && !rc; i++) h[nblk + 1 + fill[BLOCK(i)]++] = i;
 #undef BLOCK
     if (!rc) rc = awefd__res_grow(&r->rec, bytes);
-    hipError_t e = rc ? hipSuccess : awefd__copy(r->rec.p, h, bytes, hipMemcpyHostToDevice, m->stream);
+    hipError_t e = rc ? hipSuccess : awefd__copy(r->rec.p, h, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) rc = awefd__fail(AWEFD_EHIP, "resident receiver table: %s", hipGetErrorString(e));
     r->idx_off = sizeof(int) * ((size_t)nblk + 1);
     free(h);
@@ -872,7 +872,7 @@ int awefd__spher_loop(awefd_model *m, float *dtr, int jsnap, awefd_snap_fn cb, v
             hipError_t he = hipStreamSynchronize(m->stream);
             if (he == hipSuccess)
                 he = awefd__rows_down(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld,
-                                      (size_t)m->np[1] * m->np[2], m->stream);
+                                      (size_t)m->np[1] * m->np[2]);
             if (he != hipSuccess) {
                 rc = awefd__fail(AWEFD_EHIP, "snapshot copy: %s", hipGetErrorString(he));
                 break;
@@ -899,6 +899,6 @@ int awefd__spher_get_field(awefd_model *m, float *host)
 {
     HIPCHK(hipStreamSynchronize(m->stream));
     HIPCHK(awefd__rows_down(host, sizeof(float) * m->np[0], m->dC, sizeof(float) * m->ld,
-                            (size_t)m->np[1] * m->np[2], m->stream));
+                            (size_t)m->np[1] * m->np[2]));
     return AWEFD_OK;
 }
